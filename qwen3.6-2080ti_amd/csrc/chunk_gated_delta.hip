@@ -1,7 +1,10 @@
 // Chunked gated delta-rule prefill for gfx950 (dk = dv = 128, conv kernel 4,
 // chunk 64), from the raw in_proj outputs of a linear-attention layer.
 //
-// Two launches on the caller's stream (steps 1 and 2 share one grid):
+// Two launches on the caller's stream, in one of two forms chosen by the number of (row, value head)
+// pairs (kSplitHeads): prep_kernel and chunk_kernel, described here (steps 1 and 2 share one grid), or
+// for few pairs blocks_kernel and chain_kernel, the same arithmetic split at the state dependence
+// (described at blocks_kernel below).
 //  1. prep_kernel -- causal conv1d + SiLU of every q/k channel and the L2
 //     norm of q and k per (token, head), q also scaled by dk^-0.5
 //     (src/reference_ops.py:181-183, 240-258, 297-304).  Each (row, head,
@@ -49,6 +52,8 @@
 // tokens are read from the token-major K and V tiles with ds_read_b64_tr_b16.
 #include "qa_common.h"
 
+#include <type_traits>
+
 namespace qa {
 
 typedef _Float16 half_t;
@@ -71,23 +76,38 @@ constexpr int LD64 = 80;   // dwords measured to give the fewest LDS bank confli
 constexpr int PU = 3;       // tokens per prep step (the conv history length)
 constexpr int RUN = 11 * PU;  // tokens one prep wave walks (swept: 33 beats 21, 63, 66 and 129)
 
+// The split form (blocks_kernel and chain_kernel) for up to this many value heads over all rows, else prep_kernel
+// and chunk_kernel.  chunk_kernel runs two workgroups per (row, value head), each with the whole chain of its chunks
+// (about 2.5 us a chunk), so below 128 (row, value head) pairs it leaves CUs idle; the split form spreads the
+// state-independent work over all CUs and shortens the chain, at the price of writing that work's operands to HBM
+// and reading them back (36 KB per chunk and key head with two value heads, where chunk_kernel's prep writes 32).
+// Measured in us, linear_attention_prefill of 16 key heads, chunk_kernel against split: 32 pairs (one row of 32 value
+// heads) at 4096 tokens 216 : 124, at 1000 tokens 78 : 47; 64 pairs at 4096 tokens 240 : 198 (two rows of 32) and
+// 262 : 242 (four rows of 16); 96 pairs 153 : 147 at 2048 tokens and 331 : 352 at 5000; 128 pairs at 2048 173 : 186.
+constexpr int64_t kSplitHeads = 64;
+
 // ---- workspace (fp16 tensors, padded to whole chunks; tokens >= T are zero)
 struct Workspace {
+  bool split;
   int64_t tp, nch;
-  int64_t off_qn, off_kn, off_gb, bytes;
+  int64_t off_qn, off_kn, off_gb, off_rec, bytes;
 };
 
 inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t{255}; }
 
+constexpr int64_t kRecBytes = 17 * 1024;  // record of the split form per (row, value head, chunk), see REC_BYTES
+
 inline Workspace workspace_layout(int64_t batch, int64_t seq, int64_t hk, int64_t hv) {
   Workspace w{};
+  w.split = batch * hv <= kSplitHeads;
   w.nch = (seq + CH - 1) / CH;
   w.tp = w.nch * CH;
-  const int64_t qk = batch * w.tp * hk * DK * 2;  // qn, kn: (B, Tp, Hk, 128)
+  const int64_t qk = batch * w.tp * hk * DK * 2;  // qn, kn: (B, Tp, Hk, 128), or tiles per (row, key head, chunk)
   w.off_qn = 0;
   w.off_kn = align256(w.off_qn + qk);
-  w.off_gb = align256(w.off_kn + qk);  // gb: (B, Hv, Tp, 4) fp32 (G, beta, exp(G), exp(G_C - G))
-  w.bytes = align256(w.off_gb + batch * hv * w.tp * 4 * 4);
+  w.off_gb = w.off_rec = align256(w.off_kn + qk);
+  // gb: (B, Hv, Tp, 4) fp32 (G, beta, exp(G), exp(G_C - G)); rec: the records of the split form
+  w.bytes = align256(w.off_gb + (w.split ? batch * hv * w.nch * kRecBytes : batch * hv * w.tp * 4 * 4));
   return w;
 }
 
@@ -343,9 +363,9 @@ __device__ __forceinline__ h4_v tr_read(const half_t* tile, int ld, int row_g, i
 // v = hi + lo with hi = fp16(v) and lo = fp16(v - hi) (v - hi is exact in fp32).
 // lo comes from v_fma_mix{lo,hi}_f16, which take hi as an fp16 operand and
 // round the fp32 result once: 1.5 instructions per element instead of 3.5.
-// The compiler does not see these VALU writes when it inserts the wait states
-// an MFMA needs before reading a VGPR written by VALU, so the asm block ends
-// with s_nop 4.
+// The compiler does not see these VALU writes when it inserts the two wait
+// states an MFMA needs before reading a VGPR written by VALU, so the asm block
+// ends with s_nop 1.
 __device__ __forceinline__ void split4(const cfloat4& v, h4_v& hi, h4_v& lo) {
   typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
@@ -356,7 +376,7 @@ __device__ __forceinline__ void split4(const cfloat4& v, h4_v& hi, h4_v& lo) {
       "v_fma_mixhi_f16 %0, -1.0, %2, %5 op_sel:[0,1,0] op_sel_hi:[0,1,0]\n\t"
       "v_fma_mixlo_f16 %1, -1.0, %3, %6 op_sel_hi:[0,1,0]\n\t"
       "v_fma_mixhi_f16 %1, -1.0, %3, %7 op_sel:[0,1,0] op_sel_hi:[0,1,0]\n\t"
-      "s_nop 4"
+      "s_nop 1"
       : "=&v"(l0), "=&v"(l1)
       : "v"(h[0]), "v"(h[1]), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
   lo = __builtin_bit_cast(h4_v, u32x2{l0, l1});
@@ -749,11 +769,20 @@ __device__ __forceinline__ void aqk_store(unsigned char* smem, int64_t ci, int t
   store4h(Aqk + i * LD64 + aqk_col(16 * tl + 4 * lq), e[0], e[1], e[2], e[3]);
 }
 
+// Rows 16 t .. 16 t + 15 of a staged tile as the 16x16x32 operands of K S0 and S0^T Q^T (dk in kblk order).
+template <int LD>
+__device__ __forceinline__ void load_rows_s(const half_t* tile, int t, int lane, f16x8_v (&x)[DK / 32]) {
+  const int lq = lane >> 4, lc = lane & 15;
+#pragma unroll
+  for (int k = 0; k < DK / 32; ++k) x[k] = *reinterpret_cast<const f16x8_v*>(tile + (16 * t + lc) * LD + 8 * kblk(k, lq));
+}
+
 // Rows 16 t .. 16 t + 15 of a staged q or k tile as 16x16x32 operands (natural dk order).
+template <int LD = LD128>
 __device__ __forceinline__ void load_rows(const half_t* tile, int t, int lane, f16x8_v (&x)[DK / 32]) {
   const int lq = lane >> 4, lc = lane & 15;
 #pragma unroll
-  for (int k = 0; k < DK / 32; ++k) x[k] = *reinterpret_cast<const f16x8_v*>(tile + (16 * t + lc) * LD128 + 32 * k + 8 * lq);
+  for (int k = 0; k < DK / 32; ++k) x[k] = *reinterpret_cast<const f16x8_v*>(tile + (16 * t + lc) * LD + 32 * k + 8 * lq);
 }
 
 __device__ __forceinline__ cfloat4 rows_product(const f16x8_v (&x)[DK / 32], const f16x8_v (&y)[DK / 32]) {
@@ -1171,6 +1200,959 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   }
 }
 
+
+// ---------------------------------------------------------------------------
+// Split form: blocks_kernel does everything that does not depend on the state, for all chunks of all
+// heads at once on all CUs, and chain_kernel runs only the state chain, 16 or 32 dv columns to a
+// workgroup.  kSplitHeads says when, with both forms' times.
+//
+// Measured on an MI355X at one row of 6001 tokens, 16 key and 32 value heads (prep_kernel 34 us +
+// chunk_kernel 240 us there): blocks_kernel 41 us, 1.25 us a chunk for chain_kernel<1>, 118-129 us.
+// blocks_kernel is bound by HBM and VALU together: at 4 x 8192 tokens it moves 819 MB in 177 us,
+// 4.6 TB/s (224 us with 55 KB of LDS and two workgroups per CU instead of four).  chain_kernel is bound
+// by one wave's instruction issue and latencies per chunk (about 2700 cycles): timing copies without the
+// helpers' or the output waves' work run within 5%.
+//
+// Workspace record of (row, value head, chunk), REC_BYTES: the operands of the chain in the order a
+// wave reads them (16 bytes per lane, 1 KB pieces), so they are staged by plain copies:
+//   D_p diag(beta') hi | lo (4 pieces), the per-token scalars gamma', gamma, exp(G_C - G) (1 piece),
+//   -M_pk hi | lo in lower_block order (6 pieces), the six Aqk operands of the output (6 pieces).
+// k tiles are kept [row][key head][chunk][64][128], q tiles as the 16 operand pieces of Q S0.
+constexpr int REC_D = 0;
+constexpr int REC_SC = 4 * HL_BLOCK;
+constexpr int REC_M = REC_SC + 1024;
+constexpr int REC_AQK = REC_M + 6 * HL_BLOCK;
+constexpr int REC_BYTES = REC_AQK + 6 * 1024;
+static_assert(REC_BYTES == kRecBytes, "workspace layout");
+
+struct BlocksParams {
+  PrepParams c;  // qn, kn: the tiles
+  GateParams g;  // gb is not used
+  unsigned char* rec;
+};
+
+// Aqk operand n of the output product: token tile t, 32-token k-step s
+//   n:      0      1      2      3      4      5
+//   (t, s): (0,0)  (1,0)  (2,0)  (2,1)  (3,0)  (3,1)
+__device__ __forceinline__ constexpr int aqk_piece(int t, int s) { return t < 2 ? t : 2 * t - 2 + s; }
+
+__device__ __forceinline__ f16x8_v join8(const h4_v& x, const h4_v& y) {
+  return __builtin_bit_cast(f16x8_v, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// Per value head scalars of a chunk in LDS (floats): beta, G, rf, beta rf, cf (see store_gate).
+constexpr int BSC = 5 * CH;
+constexpr int B_HEADS = 4;  // value heads gated at a time (one per wave)
+constexpr int BLD = 136;                         // row stride (halfs) of the q and k tiles: four workgroups per CU
+constexpr int B_TILE = CH * BLD * 2;
+constexpr int BOFF_Q = 0;
+constexpr int BOFF_K = BOFF_Q + B_TILE;
+constexpr int BOFF_SC = BOFF_K + B_TILE;
+constexpr int B_LDS_BYTES = BOFF_SC + B_HEADS * BSC * 4;
+// over the q tile once the Gram products are in registers
+constexpr int BOFF_D = BOFF_Q;                           // D hi | lo, x 2 (by value head parity)
+constexpr int BOFF_A = BOFF_D + 2 * 4 * HL_BLOCK;        // one 16x16 fp32 block per wave
+static_assert(BOFF_A + 4 * 16 * LDB * 4 <= BOFF_K && B_LDS_BYTES <= 40 * 1024, "LDS budget");
+
+// The blocks wave U of a blocks_kernel workgroup makes.
+template <int U>
+struct BlocksWave {
+  // lower K K^T blocks (ti, tl) of this wave: first lower_block index and count
+  static constexpr int KK0 = U == 0 ? 0 : U == 1 ? 1 : U == 2 ? 3 : 5;
+  static constexpr int NKK = (U == 1 || U == 2) ? 2 : 1;
+  // Aqk operands (aqk_piece order) of this wave: 0: (0,0) (1,0); 1: (2,0); 2: (3,0); 3: (2,1) (3,1)
+  static constexpr int NAQ = (U == 0 || U == 3) ? 2 : 1;
+  static constexpr int aq_t(int i) { return U == 0 ? i : U == 1 ? 2 : U == 2 ? 3 : 2 + i; }
+  static constexpr int aq_s = U == 3 ? 1 : 0;
+};
+__device__ __forceinline__ constexpr int lb_row(int n) { return n < 1 ? 1 : n < 3 ? 2 : 3; }
+__device__ __forceinline__ constexpr int lb_col(int n) { return n - lb_row(n) * (lb_row(n) - 1) / 2; }
+
+// The state-independent operands of nr value heads of the key head, whose scalars are in LDS slots 0 .. nr - 1, by
+// wave U from its Gram products: xd = K_U K_U^T, xa its lower K K^T blocks, xq its Q K^T tiles.  rec0: the first
+// head's record, rec_step from one head's to the next.
+template <int U>
+__device__ __forceinline__ void blocks_heads(unsigned char* smem, unsigned char* rec0, int64_t rec_step, int nr, int lane,
+                                             const cfloat4& xd, const cfloat4 (&xa)[2], const cfloat4 (&xq)[2][2]) {
+  using W = BlocksWave<U>;
+  const int lq = lane >> 4, lc = lane & 15;
+  float* ab = reinterpret_cast<float*>(smem + BOFF_A) + U * 16 * LDB;
+  for (int r = 0; r < nr; ++r) {
+    const float* sc = reinterpret_cast<const float*>(smem + BOFF_SC) + r * BSC;
+    unsigned char* rec = rec0 + r * rec_step;
+    unsigned char* dl = smem + BOFF_D + (r & 1) * 4 * HL_BLOCK;
+    {
+      // A_UU from the Gram block (symmetric), then D_U = (I + A_UU)^-1
+      const int i = 16 * U + lc;
+      const float bi = sc[i];
+      const float gi = sc[CH + i];
+      const cfloat4 gl = *reinterpret_cast<const cfloat4*>(sc + CH + 16 * U + 4 * lq);
+      cfloat4 a;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = bi * __expf(gi - gl[e]) * xd[e];
+        a[e] = 4 * lq + e < lc ? v : 0.f;
+      }
+      *reinterpret_cast<cfloat4*>(ab + lc * LDB + 4 * lq) = a;
+      // one wave's LDS accesses are performed in order: the solve reads A before it writes D over it
+      solve_unit_lower16(ab, ab, lane);
+      cfloat4 dv = *reinterpret_cast<const cfloat4*>(ab + lc * LDB + 4 * lq);
+      h4_v hi, lo;
+      split4(dv, hi, lo);
+      *reinterpret_cast<f16x8_v*>(dl + U * HL_BLOCK + 16 * lane) = join8(hi, lo);
+      // the record's copy takes the columns' beta' with it: Y = D R = (D beta') (V + gamma' K S0)
+      dv *= -0.69314718055994531f * *reinterpret_cast<const cfloat4*>(sc + 16 * U + 4 * lq);
+      split4(dv, hi, lo);
+      *reinterpret_cast<f16x8_v*>(rec + REC_D + U * HL_BLOCK + 16 * lane) = join8(hi, lo);
+    }
+    lds_barrier();  // the D blocks of this head (the other parity is free: its readers are past the barrier)
+#pragma unroll
+    for (int m = 0; m < W::NKK; ++m) {
+      // -M_pk = -D_p A_pk (see m_store): A[i][l] = beta_i rf_i exp(G_{16 ti} - G_{16 tl + 15}) cf_l (K K^T)[i][l]
+      constexpr int n0 = W::KK0;
+      const int n = n0 + m;
+      const int ti = lb_row(n), tl = lb_col(n);
+      const cfloat4 brf = *reinterpret_cast<const cfloat4*>(sc + 3 * CH + 16 * ti + 4 * lq);
+      const float cs = -sc[4 * CH + 16 * tl + lc] * block_decay(sc + CH, ti, tl);
+      cfloat4 a;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = brf[e] * cs * xa[m][e];
+      h4_v ah, al;
+      split4(a, ah, al);
+      const h4_v* dsrc = reinterpret_cast<const h4_v*>(dl + ti * HL_BLOCK + 16 * lane);
+      const cfloat4 zero = {0.f, 0.f, 0.f, 0.f};
+      const cfloat4 mm = mma3(ah, al, dsrc[0], dsrc[1], zero);
+      h4_v hi, lo;
+      split4(mm, hi, lo);
+      *reinterpret_cast<f16x8_v*>(rec + REC_M + n * HL_BLOCK + 16 * lane) = join8(hi, lo);
+    }
+#pragma unroll
+    for (int m = 0; m < W::NAQ; ++m) {
+      // Aqk[i][l] = exp(G_i - G_l) (q_i . k_l), l <= i: the tiles (t, 2 s) and (t, 2 s + 1) of one operand
+      const int t = W::aq_t(m), s = W::aq_s;
+      const int i = 16 * t + lc;
+      f16x8_v o;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int tl = 2 * s + h;
+        if (tl > t) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[4 * h + e] = static_cast<half_t>(0.f);
+        } else if (tl < t) {
+          const float ri = sc[2 * CH + i] * block_decay(sc + CH, t, tl);
+          const cfloat4 cl = *reinterpret_cast<const cfloat4*>(sc + 4 * CH + 16 * tl + 4 * lq);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[4 * h + e] = static_cast<half_t>(ri * cl[e] * xq[m][h][e]);
+        } else {
+          const float gi = sc[CH + i];
+          const cfloat4 gl = *reinterpret_cast<const cfloat4*>(sc + CH + 16 * tl + 4 * lq);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float y = __expf(gi - gl[e]) * xq[m][h][e];
+            o[4 * h + e] = static_cast<half_t>(16 * tl + 4 * lq + e <= i ? y : 0.f);
+          }
+        }
+      }
+      *reinterpret_cast<f16x8_v*>(rec + REC_AQK + aqk_piece(t, s) * 1024 + 16 * lane) = o;
+    }
+  }
+}
+
+// The Gram products of wave U: xd = K_U K_U^T, xa = its lower K K^T blocks (rows ti), xq = its Q K^T tiles
+// (transposed, see aqk_store).  The wave also writes rows 16 U .. 16 U + 15 of q to the workspace in operand order
+// (piece 4 t + s of a tile: 16 bytes per lane), read into registers by the output waves.
+template <int U>
+__device__ __forceinline__ void blocks_gram(const unsigned char* smem, half_t* q_out, int lane, cfloat4& xd, cfloat4 (&xa)[2], cfloat4 (&xq)[2][2]) {
+  using W = BlocksWave<U>;
+  const half_t* Ks = reinterpret_cast<const half_t*>(smem + BOFF_K);
+  const half_t* Qs = reinterpret_cast<const half_t*>(smem + BOFF_Q);
+  f16x8_v x[DK / 32], y[DK / 32];
+  load_rows_s<BLD>(Qs, U, lane, x);
+#pragma unroll
+  for (int k = 0; k < DK / 32; ++k) *reinterpret_cast<f16x8_v*>(q_out + ((4 * U + k) * 64 + lane) * 8) = x[k];
+  load_rows<BLD>(Ks, U, lane, x);
+  xd = rows_product(x, x);
+#pragma unroll
+  for (int m = 0; m < W::NKK; ++m) {
+    load_rows<BLD>(Ks, lb_row(W::KK0 + m), lane, x);
+    load_rows<BLD>(Ks, lb_col(W::KK0 + m), lane, y);
+    xa[m] = rows_product(x, y);
+  }
+#pragma unroll
+  for (int m = 0; m < W::NAQ; ++m) {
+    load_rows<BLD>(Qs, W::aq_t(m), lane, x);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (2 * W::aq_s + h > W::aq_t(m)) continue;
+      load_rows<BLD>(Ks, 2 * W::aq_s + h, lane, y);
+      xq[m][h] = rows_product(y, x);
+    }
+  }
+}
+
+// One workgroup per (row, chunk, key head): conv1d + SiLU + L2 norm of the head's q and k rows, their Gram
+// products once, then per value head of the key head the gating and the operands D, M and Aqk.
+template <bool VEC16>
+__global__ __launch_bounds__(256, 4) void blocks_kernel(BlocksParams bp) {
+  __shared__ __align__(16) unsigned char smem[B_LDS_BYTES];
+  const PrepParams& p = bp.c;
+  const GateParams& gp = bp.g;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hk = static_cast<int>(blockIdx.x % p.Hk);
+  const int64_t rest = blockIdx.x / p.Hk;
+  const int64_t c = rest % p.nch;
+  const int64_t b = rest / p.nch;
+  const int64_t t0 = c * CH;
+  const int R = p.Hv / p.Hk;
+
+  // ---- conv + SiLU + norm: 16 lanes take eight consecutive tokens of q (even groups) or k
+  {
+    const int grp = tid >> 4;
+    const int kind = grp & 1;
+    const int run = grp >> 1;
+    const int ch = (kind * p.Hk + hk) * DK + 8 * (lane & 15);
+    const int64_t ts = t0 + 8 * run;  // first token
+    const bf16_t* xrow = p.x + b * p.x_sb + ch;
+    u32x4 raw[11];
+#pragma unroll
+    for (int j = 0; j < 11; ++j) {
+      // tokens ts - 3 .. ts + 7, clamped into the sequence (those outside are replaced below)
+      const int64_t t = max64(0, min64(ts - 3 + j, p.T - 1));
+      const bf16_t* src = xrow + t * p.x_st;
+      if constexpr (VEC16) {
+        raw[j] = *reinterpret_cast<const u32x4*>(src);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[j][e] = reinterpret_cast<const uint32_t*>(src)[e];
+      }
+    }
+    float w[8][KCONV];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float4 wc = *reinterpret_cast<const float4*>(p.conv_w + static_cast<int64_t>(ch + e) * KCONV);
+      // times -log2(e): the tap sum is t = -log2(e) a, t / (1 + 2^t) = -log2(e) silu(a), and the norm takes the
+      // constant out again
+      w[e][0] = -1.4426950408889634f * wc.x;
+      w[e][1] = -1.4426950408889634f * wc.y;
+      w[e][2] = -1.4426950408889634f * wc.z;
+      w[e][3] = -1.4426950408889634f * wc.w;
+    }
+    auto chan = [](const u32x4& r, int e) -> float {
+      const uint32_t u = r[e >> 1];
+      return __uint_as_float((e & 1) ? (u & 0xffff0000u) : (u << 16));
+    };
+    float h[3][8];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[s][e] = chan(raw[s], e);
+    if (ts == 0) {  // the tokens before the sequence: the carried conv state, or zeros
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[s][e] = p.conv_in != nullptr ? p.conv_in[(b * p.C + ch + e) * (KCONV - 1) + s] : 0.f;
+    }
+    const float scale = -0.69314718055994531f * (kind == 0 ? rsqrtf(static_cast<float>(DK)) : 1.f);
+    const bool tail = c == p.nch - 1;
+    half_t* tile = reinterpret_cast<half_t*>(smem + (kind == 0 ? BOFF_Q : BOFF_K)) + (8 * run) * BLD + 8 * (lane & 15);
+    half_t* dst = p.kn + (((b * p.Hk + hk) * p.nch + c) * CH + 8 * run) * DK + 8 * (lane & 15);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float y[8];
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float xc = chan(raw[3 + j], e);
+        const float t = w[e][0] * h[j % 3][e] + w[e][1] * h[(j + 1) % 3][e] + w[e][2] * h[(j + 2) % 3][e] + w[e][3] * xc;
+        h[j % 3][e] = xc;
+        y[e] = t * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(t));
+      }
+      if (tail && ts + j >= p.T) {  // tokens past the sequence are zero
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += y[e] * y[e];
+      constexpr float kLn2Sq = 0.48045301391820142f;
+      const float r = rsqrtf(kLn2Sq * row16_sum(ss) + 1e-6f) * scale;
+      f16x8_v o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = static_cast<half_t>(y[e] * r);
+      *reinterpret_cast<f16x8_v*>(tile + j * BLD) = o;
+      if (kind == 1) *reinterpret_cast<f16x8_v*>(dst + j * DK) = o;
+    }
+  }
+  // conv state of the head's q and k channels: the raw inputs of the last three tokens
+  if (p.conv_out != nullptr && c == p.nch - 1) {
+    const int64_t ch = static_cast<int64_t>((tid < DK ? 0 : p.Hk) + hk) * DK + (tid & (DK - 1));
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const int64_t t = p.T - 3 + s;
+      float val = 0.f;
+      if (t >= 0)
+        val = bf16_to_f32(p.x[b * p.x_sb + t * p.x_st + ch]);
+      else if (p.conv_in != nullptr)
+        val = p.conv_in[(b * p.C + ch) * (KCONV - 1) + (KCONV - 1) + t];
+      p.conv_out[(b * p.C + ch) * (KCONV - 1) + s] = val;
+    }
+  }
+
+  const int64_t rec_step = p.nch * REC_BYTES;  // from one value head to the next
+  unsigned char* rec_hk = bp.rec + ((b * p.Hv + static_cast<int64_t>(hk) * R) * p.nch + c) * REC_BYTES;
+  auto gate = [&](int r) {  // value head r of the key head: the scalars of its chunk
+    const int hv = hk * R + r;
+    const int64_t t = t0 + lane;
+    float g = 0.f, beta = 0.f;
+    if (t < p.T) {
+      const int64_t off = b * gp.ab_sb + t * gp.ab_st + hv;
+      const float a = load_ab(gp.a, gp.ab_dtype, off);
+      const float bv = load_ab(gp.bb, gp.ab_dtype, off);
+      g = -__expf(gp.a_log[hv]) * softplus_ref(a + gp.dt_bias[hv]);
+      beta = 1.f / (1.f + __expf(-bv));
+    }
+    float G = g;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float up = __shfl_up(G, off, 64);
+      if (lane >= off) G += up;
+    }
+    const float gC = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, G), CH - 1));
+    const float rf = __expf(G - __shfl(G, lane & ~15, 64));
+    const float cf = __expf(__shfl(G, lane | 15, 64) - G);
+    const float gamma = __expf(G);
+    float* sc = reinterpret_cast<float*>(smem + BOFF_SC) + (r % B_HEADS) * BSC;
+    sc[lane] = beta;
+    sc[CH + lane] = G;
+    sc[2 * CH + lane] = rf;
+    sc[3 * CH + lane] = beta * rf;
+    sc[4 * CH + lane] = cf;
+    float* gs = reinterpret_cast<float*>(rec_hk + r * rec_step + REC_SC);
+    gs[lane] = 1.4426950408889634f * gamma;  // gamma' (see conv_v for the factor)
+    gs[CH + lane] = gamma;
+    gs[2 * CH + lane] = __expf(gC - G);
+  };
+  if (wave < R) gate(wave);
+  lds_barrier();
+  half_t* q_out = p.qn + ((b * p.Hk + hk) * p.nch + c) * (CH * DK);
+  cfloat4 xd, xa[2], xq[2][2];
+  if (wave == 0) blocks_gram<0>(smem, q_out, lane, xd, xa, xq);
+  else if (wave == 1) blocks_gram<1>(smem, q_out, lane, xd, xa, xq);
+  else if (wave == 2) blocks_gram<2>(smem, q_out, lane, xd, xa, xq);
+  else blocks_gram<3>(smem, q_out, lane, xd, xa, xq);
+  lds_barrier();  // the q tile's space is free
+  for (int r0 = 0; r0 < R; r0 += B_HEADS) {
+    if (r0 > 0) {
+      lds_barrier();  // every wave is past the scalars and operands of the heads before
+      if (r0 + wave < R) gate(r0 + wave);
+      lds_barrier();
+    }
+    const int nr = min(B_HEADS, R - r0);
+    unsigned char* rec0 = rec_hk + r0 * rec_step;
+    if (wave == 0) blocks_heads<0>(smem, rec0, rec_step, nr, lane, xd, xa, xq);
+    else if (wave == 1) blocks_heads<1>(smem, rec0, rec_step, nr, lane, xd, xa, xq);
+    else if (wave == 2) blocks_heads<2>(smem, rec0, rec_step, nr, lane, xd, xa, xq);
+    else blocks_heads<3>(smem, rec0, rec_step, nr, lane, xd, xa, xq);
+  }
+}
+
+// The state chain.  Workgroup: NC slices of 16 dv columns of one (row, value head); NC chain waves, NC output
+// waves and NHW helper waves, each role with its own chunk loop and the same two barriers per chunk:
+//   phase A of chunk i: chain -- fp16 copy of S0 (also to LDS), K S0, Y = D R; output -- Aqk delta of chunk i - 1
+//     and its stores; helpers -- k tile, D and M blocks and scalars of chunk i + 1 into LDS;
+//   phase B: chain -- substitution, delta to LDS, state update; output -- gamma (S0^T Q^T); helpers -- v channels of
+//     chunk i + 1.
+// What one phase writes no other role reads in that phase: the tiles the helpers write are double-buffered by chunk
+// parity, the fp16 copies of S0 and delta are written in one phase and read in the next.  q and Aqk have one reader,
+// so they go from the workspace to its registers without LDS (a CU writes LDS at about 70 bytes a cycle).
+
+// Chunks whose pieces the helper and output waves hold in registers ahead of their use: the loads come from the
+// Infinity Cache or HBM, whose latency under load is longer than one chunk's period.
+constexpr int kAheadChunks = 2;
+
+template <int NC>
+struct Chain {
+  static_assert(NC == 1 || NC == 2, "slices per workgroup");
+  static constexpr int NHW = 4;              // helper waves
+  // with NC = 1 the wave that would share the chain wave's SIMD (index 4) ends at once
+  static constexpr int NT = 64 * (NC == 1 ? 7 : 2 * NC + NHW);
+  static constexpr int LDV = 16 * NC + 16;   // row stride (halfs) of a V tile
+  static constexpr int VB = CH * LDV * 2;
+  static constexpr int K = 0;                  // x 2
+  static constexpr int SC = K + 2 * KS_BYTES;  // x 2: gamma', gamma, dec
+  static constexpr int D = SC + 2 * 1024;      // x 2
+  static constexpr int M = D + 2 * 4 * HL_BLOCK;  // x 2
+  static constexpr int V = M + 2 * 6 * HL_BLOCK;  // x 2
+  static constexpr int SB = V + 2 * VB;        // fp16 S0 operands, 4 KB per slice
+  static constexpr int DA = SB + NC * 4096;    // fp16 delta operands, 2 KB per slice
+  static constexpr int BYTES = DA + NC * 2048;
+  static_assert(BYTES <= 160 * 1024, "LDS budget");
+  static constexpr int NK = 16 / NHW;          // k tile pieces per helper wave
+  static constexpr int ND = (5 + NHW - 1) / NHW;  // D and scalar pieces
+  static constexpr int NM = (6 + NHW - 1) / NHW;  // M pieces
+  // v conv: each helper wave takes 16 of the chunk's tokens and all 16 NC channels, a lane TG tokens of two
+  static constexpr int PAIRS = 8 * NC;
+  static constexpr int TG = 2 * NC;
+};
+
+struct ChainParams {
+  const half_t* qn;
+  const half_t* kn;
+  const unsigned char* rec;
+  const bf16_t* x;
+  int64_t x_sb, x_st;
+  const float* conv_w;
+  const float* conv_in;
+  float* conv_out;
+  int C;
+  const float* state_in;
+  float* state_out;
+  void* out;
+  int out_dtype;
+  int64_t out_sb, out_st;
+  int64_t T, nch;
+  int Hk, Hv;
+};
+
+// pieces j * NHW + h (j = 0 .. N - 1; those past `count` load the last one again and are not written) of a
+// region of 1 KB pieces
+template <int NHW, int N>
+__device__ __forceinline__ void load_pieces(const unsigned char* base, int count, int h, int lane, u32x4 (&r)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) r[j] = *reinterpret_cast<const u32x4*>(base + min(j * NHW + h, count - 1) * 1024 + 16 * lane);
+}
+
+template <int NHW, int N>
+__device__ __forceinline__ void store_pieces(unsigned char* dst, int count, int h, int lane, const u32x4 (&r)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    if (j * NHW + h < count) *reinterpret_cast<u32x4*>(dst + (j * NHW + h) * 1024 + 16 * lane) = r[j];
+}
+
+// tile pieces: piece p holds rows 4 p .. 4 p + 3 of the [64][128] tile
+template <int NHW, int N>
+__device__ __forceinline__ void store_tile(unsigned char* tile, int h, int lane, const u32x4 (&r)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    *reinterpret_cast<u32x4*>(tile + (4 * (j * NHW + h) + (lane >> 4)) * (LD128 * 2) + 16 * (lane & 15)) = r[j];
+}
+
+// A 16x16 fp32 block as the B operand of products with hi | lo blocks: its fp16 high half twice, and the rest twice.
+// block * x = mma_hh + mma_ll, two 16x16x32 products of (hi | lo) against (h, h) and (l, l), where mma3 takes three
+// products.  (hi against l alone would be a 16x16x16 product, but a chain of the two shapes on one accumulator gives
+// wrong sums on gfx950 unless wait states stand between them, and the compiler places none.)
+struct HiLo {
+  f16x8_v hh, ll;
+};
+
+__device__ __forceinline__ void split_b(const cfloat4& v, HiLo& x) {
+  h4_v h, l;
+  split4(v, h, l);
+  x.hh = join8(h, h);
+  x.ll = join8(l, l);
+}
+
+__device__ __forceinline__ cfloat4 mma_hh(const f16x8_v& hl, const HiLo& x, const cfloat4& acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(hl, x.hh, acc, 0, 0, 0);
+}
+__device__ __forceinline__ cfloat4 mma_ll(const f16x8_v& hl, const HiLo& x, const cfloat4& acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(hl, x.ll, acc, 0, 0, 0);
+}
+
+template <int NC>
+__device__ __forceinline__ void chain_role(const ChainParams& p, unsigned char* smem, int64_t b, int hv, int col0, int v, int lane) {
+  using C = Chain<NC>;
+  const int lq = lane >> 4, lc = lane & 15;
+  // state columns dv = col0 + lc as eight 16x16 tiles: S[d][r] = S[dk_of(d, 4 lq + r)][col0 + lc]
+  cfloat4 S[8];
+  const int64_t plane = (b * p.Hv + hv) * DK * DV + col0 + lc;
+#pragma unroll
+  for (int d = 0; d < 8; ++d)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[d][r] = p.state_in == nullptr ? 0.f : p.state_in[plane + static_cast<int64_t>(dk_of(d, 4 * lq + r)) * DV];
+  unsigned char* sb_l = smem + C::SB + v * 4096 + 16 * lane;
+  unsigned char* da_l = smem + C::DA + v * 2048 + 16 * lane;
+  // One wave's chain of dependent work is what a chunk costs (its instruction issue and latencies, not any unit's
+  // throughput), so operands are read from LDS well ahead of their use: kr, the K operands, during the substitution
+  // of the chunk before.
+  f16x8_v kr[4][DK / 32];
+  auto load_kr = [&](int64_t ci, int t, int s) {
+    const half_t* Ks = reinterpret_cast<const half_t*>(smem + C::K + (ci & 1) * KS_BYTES);
+    kr[t][s] = *reinterpret_cast<const f16x8_v*>(Ks + (16 * t + lc) * LD128 + 8 * kblk(s, lq));
+  };
+  auto load_gam = [&](int64_t ci) { return reinterpret_cast<const float*>(smem + C::SC + (ci & 1) * 1024)[2 * CH - 1]; };
+  float gamC = 0.f;
+  lds_barrier();
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) load_kr(0, t, s);
+  gamC = load_gam(0);
+  for (int64_t ci = 0; ci < p.nch; ++ci) {
+    const half_t* Ks = reinterpret_cast<const half_t*>(smem + C::K + (ci & 1) * KS_BYTES);
+    const half_t* Vs = reinterpret_cast<const half_t*>(smem + C::V + (ci & 1) * C::VB);
+    const float* sc = reinterpret_cast<const float*>(smem + C::SC + (ci & 1) * 1024);
+    const unsigned char* Ds = smem + C::D + (ci & 1) * 4 * HL_BLOCK + 16 * lane;
+    const unsigned char* Ms = smem + C::M + (ci & 1) * 6 * HL_BLOCK + 16 * lane;
+    h4_v v4[4];
+    f16x8_v dm[4], mm[6];  // D and M blocks, hi | lo
+    cfloat4 gm[4];
+    auto load_v = [&](int t) { v4[t] = tr_read(Vs, C::LDV, 16 * t + 4 * lq, 16 * v, lane); };
+    auto load_gm = [&](int t) { gm[t] = *reinterpret_cast<const cfloat4*>(sc + 16 * t + 4 * lq); };
+    auto load_d = [&](int t) { dm[t] = *reinterpret_cast<const f16x8_v*>(Ds + t * HL_BLOCK); };
+    auto load_m = [&](int n) { mm[n] = *reinterpret_cast<const f16x8_v*>(Ms + n * HL_BLOCK); };
+    // ---- phase A: K S0, then Y_t = D_t diag(beta') (V + gamma' K S0), which is D R with R = beta (v - gamma K S0)
+    // and V = -log2(e) v
+    f16x8_v sb[DK / 32];
+    cfloat4 Y[4], acc[4];
+    auto make_r = [&](int t, HiLo& x) {
+      cfloat4 R;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) R[r] = __builtin_fmaf(gm[t][r], acc[t][r], static_cast<float>(v4[t][r]));
+      split_b(R, x);
+    };
+    f16x8_v ka[2][8];
+    HiLo x0, x1, x2;  // delta_p
+    const cfloat4 zero = {0.f, 0.f, 0.f, 0.f};
+    // Pairs of token tiles follow each other through the products, so the dependent VALU work of one pair (about
+    // ten cycles an instruction) runs beside the products of the next; the LDS accesses go beside products too.
+    auto put_sb = [&](int s) { *reinterpret_cast<f16x8_v*>(sb_l + 1024 * s) = sb[s]; };
+    auto ks = [&](int t, int s) { acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kr[t][s], sb[s], acc[t], 0, 0, 0); };
+    HiLo x[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = zero;
+    sb[0] = pack8h(S[0], S[1]);
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) {
+      ks(0, s);
+      if (s < 3) sb[s + 1] = pack8h(S[2 * s + 2], S[2 * s + 3]);
+      ks(1, s);
+      put_sb(s);
+      if (s < 2) {
+        load_gm(s);
+        load_v(s);
+        load_d(s);
+      }
+    }
+    make_r(0, x[0]);
+    make_r(1, x[1]);
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) {
+      ks(2, s);
+      ks(3, s);
+    }
+#pragma unroll
+    for (int t = 2; t < 4; ++t) {
+      load_gm(t);
+      load_v(t);
+      load_d(t);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) ka[0][d] = ktr_operand(Ks, 4 * lq, d, lane);
+    make_r(2, x[2]);
+    make_r(3, x[3]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) Y[t] = mma_hh(dm[t], x[t], zero);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) Y[t] = mma_ll(dm[t], x[t], Y[t]);
+#pragma unroll
+    for (int d = 4; d < 8; ++d) ka[0][d] = ktr_operand(Ks, 4 * lq, d, lane);
+#pragma unroll
+    for (int t = 2; t < 4; ++t) Y[t] = mma_hh(dm[t], x[t], zero);
+#pragma unroll
+    for (int n = 0; n < 6; ++n) load_m(n);
+    split_b(Y[0], x0);
+#pragma unroll
+    for (int t = 2; t < 4; ++t) Y[t] = mma_ll(dm[t], x[t], Y[t]);
+    // half of the state's decay over the chunk (the rest beside the first products of phase B)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) S[d] *= gamC;
+    lds_barrier();
+    // ---- phase B: delta_p = Y_p - sum_{k<p} M_pk delta_k (the blocks are stored as -M, so delta accumulates in
+    // Y), then S += K^T (dec delta)
+    cfloat4 de[4];
+    auto load_de = [&](int t) { de[t] = *reinterpret_cast<const cfloat4*>(sc + 2 * CH + 16 * t + 4 * lq); };
+    auto half_bd = [&](int t) -> h4_v {  // dec delta of token tile t, fp16
+      h4_v r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = static_cast<half_t>(de[t][e] * Y[t][e]);
+      return r;
+    };
+    auto put_da = [&](int s) { *reinterpret_cast<f16x8_v*>(da_l + 1024 * s) = pack8h(Y[2 * s], Y[2 * s + 1]); };
+    // LDS accesses that go beside the products, one each: dec, the second half of K^T, chunk ci + 1's K operands
+    // (its tile is complete; past the last chunk a stale one, never used) and its decay
+    auto side = [&](int k) {
+      if (k < 4) load_de(k);
+      else if (k < 12) ka[1][k - 4] = ktr_operand(Ks, 32 + 4 * lq, k - 4, lane);
+      else if (k < 28) load_kr(ci + 1, (k - 12) & 3, (k - 12) >> 2);
+    };
+    f16x8_v bd0, bd1;
+    auto hh = [&](int q, int n, const HiLo& x, int k) {
+      Y[q] = mma_hh(mm[n], x, Y[q]);
+      side(k);
+    };
+    auto hl = [&](int q, int n, const HiLo& x, int k) {
+      Y[q] = mma_ll(mm[n], x, Y[q]);
+      side(k);
+    };
+    auto update = [&](int s, int d, const f16x8_v& bd, int k) {
+      S[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[s][d], bd, S[d], 0, 0, 0);
+      side(k);
+    };
+    hh(1, 0, x0, 0);  // M(1,0) and M(2,0)
+    hh(2, 1, x0, 1);
+    S[4] *= gamC;
+    hl(1, 0, x0, 2);
+    hl(2, 1, x0, 3);
+    S[5] *= gamC;
+    hh(3, 3, x0, 4);  // M(3,0)
+    split_b(Y[1], x1);
+    S[6] *= gamC;
+    hl(3, 3, x0, 5);
+    const h4_v b0 = half_bd(0);
+    hh(2, 2, x1, 6);  // M(2,1) and M(3,1)
+    hh(3, 4, x1, 7);
+    bd0 = join8(b0, half_bd(1));
+    hl(2, 2, x1, 8);
+    hl(3, 4, x1, 9);
+    S[7] *= gamC;
+    gamC = load_gam(ci + 1);
+    update(0, 0, bd0, 10);
+    split_b(Y[2], x2);
+    update(0, 1, bd0, 11);
+    update(0, 2, bd0, 12);
+    hh(3, 5, x2, 13);  // M(3,2)
+    update(0, 3, bd0, 14);
+    hl(3, 5, x2, 15);
+    update(0, 4, bd0, 16);
+    update(0, 5, bd0, 17);
+    const h4_v b2 = half_bd(2);
+    update(0, 6, bd0, 18);
+    put_da(0);
+    update(0, 7, bd0, 19);
+    bd1 = join8(b2, half_bd(3));
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      update(1, d, bd1, 20 + d);
+      if (d == 2) put_da(1);
+    }
+    lds_barrier();
+  }
+  if (p.state_out != nullptr) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p.state_out[plane + static_cast<int64_t>(dk_of(d, 4 * lq + r)) * DV] = S[d][r];
+  }
+}
+
+template <int NC>
+__device__ __forceinline__ void output_role(const ChainParams& p, unsigned char* smem, int64_t b, int hv, int qh, int col0, int v, int lane) {
+  using C = Chain<NC>;
+  const int lq = lane >> 4, lc = lane & 15, odd = lq & 1;
+  const unsigned char* sb_l = smem + C::SB + v * 4096 + 16 * lane;
+  const unsigned char* da_l = smem + C::DA + v * 2048 + 16 * lane;
+  const bool out16 = p.out_dtype == QA_BF16 && p.out_st % 8 == 0 && p.out_sb % 8 == 0;
+  // q and Aqk operands, straight from the workspace: kAheadChunks ahead in registers (set i % 2 holds chunk i)
+  const int64_t last = p.nch - 1;
+  const unsigned char* qt = reinterpret_cast<const unsigned char*>(p.qn) + (b * p.Hk + qh) * p.nch * (CH * DK * 2) + 16 * lane;
+  const unsigned char* rc = p.rec + (b * p.Hv + hv) * p.nch * REC_BYTES + REC_AQK + 16 * lane;
+  f16x8_v qo[kAheadChunks][16], ao[kAheadChunks][6];
+  auto load_q = [&](int64_t ci, int u) {
+#pragma unroll
+    for (int n = 0; n < 16; ++n) qo[u][n] = *reinterpret_cast<const f16x8_v*>(qt + ci * (CH * DK * 2) + 1024 * n);
+  };
+  auto load_aq = [&](int64_t ci, int u) {
+#pragma unroll
+    for (int n = 0; n < 6; ++n) ao[u][n] = *reinterpret_cast<const f16x8_v*>(rc + ci * REC_BYTES + 1024 * n);
+  };
+#pragma unroll
+  for (int i = 0; i < kAheadChunks; ++i) {
+    load_q(min64(i, last), i);
+    load_aq(min64(i, last), i);
+  }
+  cfloat4 On[4];
+  lds_barrier();
+  auto finish = [&](int64_t ci, int u) {  // chunk ci - 1 (set u): Aqk delta and the stores
+    {
+      f16x8_v da[2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) da[s] = *reinterpret_cast<const f16x8_v*>(da_l + 1024 * s);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (s == 1 && t < 2) continue;
+          On[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(da[s], ao[u][aqk_piece(t, s)], On[t], 0, 0, 0);
+        }
+      const int64_t tc0 = (ci - 1) * CH;
+      const int ntok = static_cast<int>(min64(CH, p.T - tc0));
+      const int64_t obase = b * p.out_sb + tc0 * p.out_st + static_cast<int64_t>(hv) * DV + col0;
+      if (out16) {
+        // 16-byte stores: see key_phase_b
+        bf16_t* o16 = reinterpret_cast<bf16_t*>(p.out) + obase;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          float lo[4], hi[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(On[2 * m][r]), __float_as_uint(On[2 * m + 1][r]), false, false);
+            lo[r] = __uint_as_float(sw[0]);
+            hi[r] = __uint_as_float(sw[1]);
+          }
+          const int tok = 16 * (2 * m + odd) + lc;
+          if (tok < ntok) {
+            uint4 packed;
+            packed.x = static_cast<uint32_t>(f32_to_bf16(lo[0])) | (static_cast<uint32_t>(f32_to_bf16(lo[1])) << 16);
+            packed.y = static_cast<uint32_t>(f32_to_bf16(lo[2])) | (static_cast<uint32_t>(f32_to_bf16(lo[3])) << 16);
+            packed.z = static_cast<uint32_t>(f32_to_bf16(hi[0])) | (static_cast<uint32_t>(f32_to_bf16(hi[1])) << 16);
+            packed.w = static_cast<uint32_t>(f32_to_bf16(hi[2])) | (static_cast<uint32_t>(f32_to_bf16(hi[3])) << 16);
+            *reinterpret_cast<uint4*>(o16 + static_cast<uint32_t>(tok) * static_cast<uint32_t>(p.out_st) + 4 * (lq - odd)) = packed;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int tok = 16 * t + lc;
+          if (tok < ntok) {
+            const int64_t o = obase + tok * p.out_st + 4 * lq;
+            if (p.out_dtype == QA_BF16) {
+              uint2 packed;
+              packed.x = static_cast<uint32_t>(f32_to_bf16(On[t][0])) | (static_cast<uint32_t>(f32_to_bf16(On[t][1])) << 16);
+              packed.y = static_cast<uint32_t>(f32_to_bf16(On[t][2])) | (static_cast<uint32_t>(f32_to_bf16(On[t][3])) << 16);
+              *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.out) + o) = packed;
+            } else {
+              *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + o) = make_float4(On[t][0], On[t][1], On[t][2], On[t][3]);
+            }
+          }
+        }
+      }
+    }
+  };
+  auto step = [&](int64_t ci, int u, int u1) {  // u: the set of chunk ci, u1: of chunk ci - 1
+    // ---- phase A
+    if (ci > 0) finish(ci, u1);
+    load_aq(min64(ci - 1 + kAheadChunks, last), u1);
+    lds_barrier();
+    // ---- phase B: gamma (S0^T Q^T) of chunk ci
+    const float* sc = reinterpret_cast<const float*>(smem + C::SC + (ci & 1) * 1024);
+    f16x8_v sb[DK / 32];
+    float gam[4];
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) sb[s] = *reinterpret_cast<const f16x8_v*>(sb_l + 1024 * s);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      gam[t] = sc[CH + 16 * t + lc];
+      On[t] = cfloat4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) On[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sb[s], qo[u][4 * t + s], On[t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) On[t] *= gam[t];
+    load_q(min64(ci + kAheadChunks, last), u);
+    lds_barrier();
+  };
+  static_assert(kAheadChunks == 2, "two register sets, by chunk parity");
+  for (int64_t ci = 0; ci < p.nch; ci += 2) {
+    step(ci, 0, 1);
+    if (ci + 1 < p.nch) step(ci + 1, 1, 0);
+  }
+  if (p.nch & 1)
+    finish(p.nch, 0);
+  else
+    finish(p.nch, 1);
+}
+
+template <int NC>
+__device__ __forceinline__ void helper_role(const ChainParams& p, unsigned char* smem, int64_t b, int hv, int qh, int col_wg, int h, int lane) {
+  using C = Chain<NC>;
+  constexpr int NHW = C::NHW, TG = C::TG;
+  const int64_t last = p.nch - 1;
+  const unsigned char* kt = reinterpret_cast<const unsigned char*>(p.kn) + (b * p.Hk + qh) * p.nch * (CH * DK * 2);
+  const unsigned char* rc = p.rec + (b * p.Hv + hv) * p.nch * REC_BYTES;
+
+  // ---- v conv: this wave convolves tokens 16 h .. 16 h + 15 of each chunk, this lane TG of them from tok0 in
+  // the channels vch and vch + 1.  Three more rows before its tokens give the conv's history.
+  const int pair = lane % C::PAIRS;
+  const int tok0 = 16 * h + TG * (lane / C::PAIRS);
+  const int64_t vch = 2 * static_cast<int64_t>(p.Hk) * DK + static_cast<int64_t>(hv) * DV + col_wg + 2 * pair;
+  const bf16_t* xv = p.x + b * p.x_sb + vch;
+  float w[2][KCONV];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    // times -log2(e): see conv_v
+    const float4 wc = *reinterpret_cast<const float4*>(p.conv_w + (vch + e) * KCONV);
+    w[e][0] = -1.4426950408889634f * wc.x;
+    w[e][1] = -1.4426950408889634f * wc.y;
+    w[e][2] = -1.4426950408889634f * wc.z;
+    w[e][3] = -1.4426950408889634f * wc.w;
+  }
+  uint32_t raw[kAheadChunks][TG + 3];
+  // Row 0 of the lane's window is token 64 ci + tok0 - 3; offsets count from the chunk's first token - 3, so they
+  // are 32 bits and, for a chunk inside the sequence, the same for every chunk.
+  const uint32_t xst = static_cast<uint32_t>(p.x_st);
+  auto load_v2 = [&](int64_t ci, uint32_t (&r)[TG + 3]) {
+    const int64_t first = ci * CH - (KCONV - 1);
+    const bf16_t* base = xv + first * p.x_st;
+    const int lo = first < 0 ? KCONV - 1 : 0;                                          // rows before the sequence
+    const int hi = static_cast<int>(min64(CH + KCONV - 2, p.T - 1 - first));           // and past it: clamped
+    uint32_t off[TG + 3];
+#pragma unroll
+    for (int j = 0; j < TG + 3; ++j) off[j] = static_cast<uint32_t>(tok0 + j) * xst;
+    if (lo > 0 || hi < CH + KCONV - 2) {
+#pragma unroll
+      for (int j = 0; j < TG + 3; ++j) off[j] = static_cast<uint32_t>(max(lo, min(tok0 + j, hi))) * xst;
+    }
+#pragma unroll
+    for (int j = 0; j < TG + 3; ++j) r[j] = *reinterpret_cast<const uint32_t*>(base + off[j]);
+  };
+  // first: chunk 0, whose history is the conv state (a load, so it stays out of the chunk loop: a load under a
+  // condition there would make every wait drain the pieces in flight)
+  auto conv = [&](int64_t ci, const uint32_t (&r)[TG + 3], auto first) {
+    float xf[TG + 3][2];
+#pragma unroll
+    for (int j = 0; j < TG + 3; ++j) {
+      xf[j][0] = __uint_as_float(r[j] << 16);
+      xf[j][1] = __uint_as_float(r[j] & 0xffff0000u);
+    }
+    const int64_t t0 = ci * CH + tok0 - (KCONV - 1);
+    if constexpr (decltype(first)::value) {
+#pragma unroll
+      for (int j = 0; j < TG + 3; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (t0 + j < 0) xf[j][e] = p.conv_in != nullptr ? p.conv_in[(b * p.C + vch + e) * (KCONV - 1) + (KCONV - 1) + t0 + j] : 0.f;
+    }
+    if (ci >= last) {  // tokens past the sequence enter as zeros
+#pragma unroll
+      for (int j = 0; j < TG + 3; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) xf[j][e] = t0 + j < p.T ? xf[j][e] : 0.f;
+    }
+    half_t* dst = reinterpret_cast<half_t*>(smem + C::V + (ci & 1) * C::VB) + tok0 * C::LDV + 2 * pair;
+#pragma unroll
+    for (int j = 0; j < TG; ++j) {
+      f16x2_v o;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float t = w[e][0] * xf[j][e] + w[e][1] * xf[j + 1][e] + w[e][2] * xf[j + 2][e] + w[e][3] * xf[j + 3][e];
+        o[e] = static_cast<half_t>(t * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(t)));
+      }
+      *reinterpret_cast<f16x2_v*>(dst + j * C::LDV) = o;
+    }
+  };
+
+  // ---- registers of the pieces of the next chunks: set i % 2 holds chunk i's; each is loaded again as soon as it
+  // is in LDS
+  u32x4 rk[kAheadChunks][C::NK], rd[kAheadChunks][C::ND], rm[kAheadChunks][C::NM];
+  constexpr int64_t TILE = CH * DK * 2;
+  auto load_kdm = [&](int64_t ci, int u) {
+    load_pieces<NHW>(kt + ci * TILE, 16, h, lane, rk[u]);
+    load_pieces<NHW>(rc + ci * REC_BYTES + REC_D, 5, h, lane, rd[u]);
+    load_pieces<NHW>(rc + ci * REC_BYTES + REC_M, 6, h, lane, rm[u]);
+  };
+  auto store_kdm = [&](int64_t ci, int u) {
+    store_tile<NHW>(smem + C::K + (ci & 1) * KS_BYTES, h, lane, rk[u]);
+    // pieces 0..3 are D, piece 4 the scalars
+#pragma unroll
+    for (int j = 0; j < C::ND; ++j) {
+      const int n = j * NHW + h;
+      if (n < 4)
+        *reinterpret_cast<u32x4*>(smem + C::D + ((ci & 1) * 4 + n) * 1024 + 16 * lane) = rd[u][j];
+      else if (n == 4)
+        *reinterpret_cast<u32x4*>(smem + C::SC + (ci & 1) * 1024 + 16 * lane) = rd[u][j];
+    }
+    store_pieces<NHW>(smem + C::M + (ci & 1) * 6 * HL_BLOCK, 6, h, lane, rm[u]);
+  };
+#pragma unroll
+  for (int i = 0; i < kAheadChunks; ++i) {
+    load_v2(min64(i, last), raw[i]);
+    load_kdm(min64(i, last), i);
+  }
+  conv(0, raw[0], std::true_type{});
+  load_v2(min64(kAheadChunks, last), raw[0]);
+  store_kdm(0, 0);
+  load_kdm(min64(kAheadChunks, last), 0);
+  lds_barrier();
+  auto step = [&](int64_t ci, int u) {  // u: the set of chunk ci + 1
+    // ---- phase A
+    store_kdm(ci + 1, u);
+    load_kdm(min64(ci + 1 + kAheadChunks, last), u);
+    lds_barrier();
+    // ---- phase B
+    conv(ci + 1, raw[u], std::false_type{});
+    load_v2(min64(ci + 1 + kAheadChunks, last), raw[u]);
+    lds_barrier();
+  };
+  for (int64_t ci = 0; ci < p.nch; ci += 2) {
+    step(ci, 1);
+    if (ci + 1 < p.nch) step(ci + 1, 0);
+  }
+  if (p.conv_out != nullptr) {
+    ChunkParams vp{};  // the fields conv_tail reads
+    vp.x = p.x;
+    vp.x_sb = p.x_sb;
+    vp.x_st = p.x_st;
+    vp.conv_in = p.conv_in;
+    vp.conv_out = p.conv_out;
+    vp.C = p.C;
+    vp.T = p.T;
+    for (int n = h; n < 2 * NC; n += NHW) conv_tail<8>(vp, b, vch - 2 * pair + 8 * n, lane);
+  }
+}
+
+template <int NC>
+__global__ __launch_bounds__(Chain<NC>::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void chain_kernel(ChainParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroup -> (row, value head, 16 NC columns); the workgroups of one key head on one XCD (see chunk_item)
+  const int per = p.Hv / p.Hk;
+  constexpr int SL = 8 / NC;
+  const int members = SL * per;
+  const int groups = static_cast<int>(gridDim.x) / members;
+  const int bid = static_cast<int>(blockIdx.x);
+  int g, r;
+  if (groups % 8 == 0) {
+    const int s = bid >> 3;
+    g = (bid & 7) + 8 * (s / members);
+    r = s % members;
+  } else {
+    g = bid / members;
+    r = bid % members;
+  }
+  const int64_t b = g / p.Hk;
+  const int qh = g % p.Hk;
+  const int hv = qh * per + r / SL;
+  const int col_wg = (r % SL) * 16 * NC;
+  if (wave < NC) {
+    __builtin_amdgcn_s_setprio(3);
+    chain_role<NC>(p, smem, b, hv, col_wg + 16 * wave, wave, lane);
+  } else if (wave < 2 * NC) {
+    output_role<NC>(p, smem, b, hv, qh, col_wg + 16 * (wave - NC), wave - NC, lane);
+  } else {
+    if (NC == 1 && wave == 4) return;
+    const int h = NC == 1 && wave > 4 ? wave - 3 : wave - 2 * NC;
+    helper_role<NC>(p, smem, b, hv, qh, col_wg, h, lane);
+  }
+}
+
+template <int NC>
+static int launch_chain(const ChainParams& p, int64_t slices, hipStream_t stream) {
+  static bool attr_set = false;  // per instantiation
+  if (!attr_set) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&chain_kernel<NC>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, Chain<NC>::BYTES);
+    if (err != hipSuccess) return fail("chunk_gated_delta_rule: cannot reserve %d bytes of LDS: %s", Chain<NC>::BYTES, hipGetErrorString(err));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((chain_kernel<NC>), dim3(static_cast<unsigned>(slices / NC)), dim3(Chain<NC>::NT), Chain<NC>::BYTES, stream, p);
+  return 0;
+}
+
 }  // namespace cgd
 }  // namespace qa
 
@@ -1248,6 +2230,49 @@ extern "C" int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype,
   const int64_t gate_waves = batch * value_heads * ws.nch;
   QA_REQUIRE(prep_waves + gate_waves <= 4 * static_cast<int64_t>(0x7fffffff), "chunk_gated_delta_rule: too many prep waves");
   const bool vec16 = x_stride_t % 8 == 0 && x_stride_b % 8 == 0 && (reinterpret_cast<uintptr_t>(mixed_qkv) & 15u) == 0;
+  if (ws.split) {
+    BlocksParams bp{};
+    bp.c = pp;
+    bp.g = gp;
+    bp.rec = wsb + ws.off_rec;
+    {
+      KernelTimer timer_("chunk_prep", stream);
+      const dim3 grid(static_cast<unsigned>(batch * ws.nch * key_heads));
+      if (vec16)
+        hipLaunchKernelGGL(blocks_kernel<true>, grid, dim3(256), 0, stream, bp);
+      else
+        hipLaunchKernelGGL(blocks_kernel<false>, grid, dim3(256), 0, stream, bp);
+    }
+    if (int rc = check_launch("chunk_gated_delta_rule blocks")) return rc;
+    ChainParams cp{};
+    cp.qn = pp.qn;
+    cp.kn = pp.kn;
+    cp.rec = bp.rec;
+    cp.x = pp.x;
+    cp.x_sb = x_stride_b;
+    cp.x_st = x_stride_t;
+    cp.conv_w = conv_weight;
+    cp.conv_in = conv_state_in;
+    cp.conv_out = conv_state_out;
+    cp.C = C;
+    cp.state_in = initial_state;
+    cp.state_out = final_state;
+    cp.out = out;
+    cp.out_dtype = out_dtype;
+    cp.out_sb = out_stride_b;
+    cp.out_st = out_stride_t;
+    cp.T = seq;
+    cp.nch = ws.nch;
+    cp.Hk = key_heads;
+    cp.Hv = value_heads;
+    const int64_t slices = batch * value_heads * 8;
+    {
+      KernelTimer timer_("chunk_gated_delta", stream);
+      // one 16-column slice per workgroup while that keeps every CU to one workgroup, else two
+      if (int rc = slices <= 256 ? launch_chain<1>(cp, slices, stream) : launch_chain<2>(cp, slices, stream)) return rc;
+    }
+    return check_launch("chunk_gated_delta_rule");
+  }
   {
     // conv + SiLU + norms, with the gating (g, beta and the in-chunk cumulative G) as extra waves
     KernelTimer timer_("chunk_prep", stream);

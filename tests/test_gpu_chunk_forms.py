@@ -1,0 +1,59 @@
+"""Both forms of the chunked delta rule and both widths of the split form's workgroups, at their edges.
+
+The number of (row, value head) pairs picks the form: up to 32 pairs one 16-column slice per
+workgroup, up to 64 two, above that ``chunk_kernel``.  Each at sequence lengths around the conv
+history (3 tokens) and the 64-token chunk, with odd and even chunk counts, with and without
+carried states, and with token rows that are only 4-byte aligned.  Tolerances as in
+``test_gpu_chunk_gated_delta``: outputs 2e-2, fp32 state 1e-3 relative, conv state bit-exact.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import gated_delta as gd
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _case(batch: int, key_heads: int, value_heads: int, seq: int, carried: bool, aligned: bool, out_dtype: torch.dtype) -> None:
+    import hip_ops
+
+    shape = gd.LinearShape(key_heads, value_heads, 128, 128, 4)
+    gen = torch.Generator().manual_seed(1000 * batch + 10 * value_heads + seq)
+    mixed = torch.randn(batch, seq, shape.qkv_dim, generator=gen).to(torch.bfloat16)
+    a = torch.randn(batch, seq, value_heads, generator=gen)
+    b = torch.randn(batch, seq, value_heads, generator=gen)
+    a_log = torch.randn(value_heads, generator=gen) - 1.0
+    dt_bias = 0.1 * torch.randn(value_heads, generator=gen)
+    w = torch.randn(shape.qkv_dim, 1, 4, generator=gen) * 0.5
+    tail = torch.randn(batch, shape.qkv_dim, 3, generator=gen) if carried else None
+    state = 0.05 * torch.randn(batch, value_heads, 128, 128, generator=gen) if carried else None
+    ref, ref_state, ref_tail = gd.linear_attention_core(mixed.float(), a, b, a_log, dt_bias, w, shape, conv_tail=tail, initial_state=state)
+    x = mixed.to(DEV)
+    if not aligned:  # rows start 4 bytes past a 16-byte boundary
+        wide = torch.zeros(batch, seq, shape.qkv_dim + 4, dtype=torch.bfloat16, device=DEV)
+        wide[..., 2 : 2 + shape.qkv_dim] = x
+        x = wide[..., 2 : 2 + shape.qkv_dim]
+    out, new_state, new_tail = hip_ops.chunk_gated_delta_rule(
+        x, a.to(DEV), b.to(DEV), a_log.to(DEV), dt_bias.to(DEV), w.to(DEV), key_heads=key_heads, value_heads=value_heads,
+        conv_state=None if tail is None else tail.to(DEV), initial_state=None if state is None else state.to(DEV), out_dtype=out_dtype)
+    torch.testing.assert_close(out.cpu().float(), ref, atol=2e-2, rtol=2e-2)
+    err = float((new_state.double().cpu() - ref_state.double()).norm() / ref_state.double().norm())
+    assert err < 1e-3, err
+    torch.testing.assert_close(new_tail.cpu(), ref_tail, atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("batch,key_heads,value_heads", [(1, 1, 1), (1, 1, 5), (2, 4, 16), (3, 1, 11), (4, 8, 16), (5, 1, 13)])
+@pytest.mark.parametrize("seq", [1, 3, 64, 65, 130])
+def test_forms_match_oracle(batch, key_heads, value_heads, seq) -> None:
+    _case(batch, key_heads, value_heads, seq, seq % 2 == 1, True, torch.bfloat16)
+
+
+@pytest.mark.parametrize("batch,key_heads,value_heads", [(1, 2, 4), (3, 4, 12)])
+@pytest.mark.parametrize("seq", [2, 63, 192, 259])
+def test_split_form_unaligned_rows_and_fp32_output(batch, key_heads, value_heads, seq) -> None:
+    _case(batch, key_heads, value_heads, seq, seq != 192, False, torch.float32)
