@@ -18,14 +18,15 @@
 // operand, so a lane's accumulator holds four consecutive outputs of one x row
 // (16-byte stores).
 //
-// Tiled path (16 rows or fewer, or more than 256): a workgroup of 4 waves owns one
+// Tiled path (16 rows or fewer, or more than 256 where the block path has too few tiles): a workgroup of 4 waves owns one
 // 128-row block of W (one scale row) for 16 * MS rows of x and a range of 128-deep
 // K blocks.  Per K block the x tile goes to LDS (double-buffered, one barrier per
 // block); each wave streams its 32 weight rows straight from global memory into
 // registers two blocks ahead.  When the grid is small, K is split over workgroups
 // that write fp32 partials, summed in a fixed order by a second kernel.  Wide path
 // (17 to 256 rows of 16-bit x): see fp8_linear_wide_kernel below, one pass over K
-// per output tile with no K split.
+// per output tile with no K split.  Block path (many output tiles): see
+// fp8_linear_block_kernel.
 #include "qa_common.h"
 
 #include <type_traits>
@@ -655,6 +656,252 @@ __global__ __launch_bounds__(WNT) void fp8_linear_xres_kernel(Params p) {
   }
 }
 
+// ---- Block path (16-bit x, more than 128 rows, see make_plan): output tiles large enough for the matrix cores to bound it.
+//
+// Work item: TM rows of x by TN weight rows by all of K, 8 waves in a WM x WN grid, each MT x NT tiles of 32 x 32
+// outputs on v_mfma_f32_32x32x16.  x (16-bit) and weight bytes go from global memory to LDS in 64-column stages
+// (global_load_lds_dwordx4) through a ring of four, three in flight.  The two waves of a SIMD (w and w + 4) work half a
+// stage apart: while one multiplies its 16 MFMAs the other reads the next operands from LDS and decodes the weights, and
+// a barrier at each change keeps them so; in step with each other both would wait for LDS at once and then both for the
+// matrix cores (4096 x 8192 x 2048: 169 us).  The copies and the scale FMAs of finished tiles are issued between the
+// MFMAs.  A tile is summed over the 128 columns of a block before the block scale multiplies it into the accumulators.
+// The copies take a uniform base and a 32-bit lane offset: with a 64-bit address per lane each one waited for the MFMAs
+// of the SIMD's other wave (129 against 65 cycles; the whole product 184 us instead of 163).
+// 16-byte pieces are XOR-swizzled by row (x: piece ^ row / 2 mod 8 of 128-byte rows, row-major weights: piece ^ row / 4
+// mod 4 of 64-byte rows; packed weights keep their order), so the lanes of one LDS access fall on distinct banks.  x is
+// the A operand: a lane's accumulators are one output column and a store instruction writes two 128-byte row pieces.
+// Workgroups go to the XCDs in contiguous ranges of tiles ordered by groups of kGroupN weight tiles, x tiles fastest
+// inside a group, so an XCD's L2 holds the group's weights while x streams.
+// What bounds it: an MFMA phase takes about 750 cycles for 520 cycles of MFMA (rows 4096, tile 128 x 256).  Measured
+// with fp32 x, its cast included (us, before: the tiled or x-resident kernels): 4096 x 8192 x 2048 208 -> 154 (895
+// TFLOP/s), 4096 x 2048 x 4096 110 -> 82, 1024 x 4096 x 2048 34.7 -> 29.4, 256 x 8192 x 2048 25.8 -> 20.6.
+typedef float f32x16_v __attribute__((ext_vector_type(16)));
+constexpr int kGroupN = 4;
+
+__device__ __forceinline__ f32x16_v mfma32(const bf16x8_v& a, const bf16x8_v& b, const f32x16_v& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16_v mfma32(const f16x8_v& a, const f16x8_v& b, const f32x16_v& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+template <int MT, int NT, int WM, int WN>
+struct BlockCfg {
+  static_assert(WM * WN == 8, "eight waves");
+  static constexpr int TM = 32 * MT * WM, TN = 32 * NT * WN;
+  static constexpr int SK = KB / 2;              // columns of a stage
+  static constexpr int kXBytes = TM * SK * 2;
+  static constexpr int kBuf = kXBytes + TN * SK;
+  static constexpr int kStages = 4;              // ring: three stages of copies in flight ahead of the one multiplied
+  static constexpr int kScaleRows = (TN + KB - 1) / KB;
+  static constexpr int kXCopies = TM / 64;       // 1 KB copies per wave and stage
+  static constexpr int kWCopies = TN / 128;
+  static constexpr int kCopies = kXCopies + kWCopies;
+  static_assert(TM % 64 == 0 && TN % 128 == 0, "whole copies per wave");
+  static int bytes(int64_t K) { return kStages * kBuf + static_cast<int>(kScaleRows * (K / KB) * 4); }
+};
+
+// lds_copy16 (see qa_common.h) from a uniform base and this lane's byte offset
+__device__ __forceinline__ void lds_copy16_at(const void* base, uint32_t offset, uint32_t lds) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, %3\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(lds), "v"(offset), "s"(base)
+      : "memory");
+}
+
+// The workgroup's barrier with nothing moved across it, register work included.
+__device__ __forceinline__ void phase_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int MODE, int MT, int NT, int WM, int WN>
+__global__ __launch_bounds__(512) void fp8_linear_block_kernel(Params p, int tiles_m, int tiles_n) {
+  static_assert(MODE == X_BF16 || MODE == X_F16, "16-bit x only");
+  typedef typename ModeTraits<MODE>::V V;
+  using C = BlockCfg<MT, NT, WM, WN>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const uint32_t smem_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // tile of this workgroup (the grid is padded to whole XCD ranges)
+  const int per_xcd = static_cast<int>(gridDim.x) >> 3;
+  const int t = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (t >= tiles_m * tiles_n) return;
+  const int grp = t / (tiles_m * kGroupN);
+  const int r = t - grp * tiles_m * kGroupN;
+  const int gw = min(kGroupN, tiles_n - grp * kGroupN);
+  const int64_t m0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(r / gw)) * C::TM;
+  const int64_t n0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(grp * kGroupN + r % gw)) * C::TN;
+  const int64_t nkb = p.K / KB;
+  const int ns = static_cast<int>(2 * nkb);  // stages
+
+  // Copy sources (rows past the ends re-read the last one and are not stored).  x copy j of wave w fills LDS rows
+  // 8 (w + 8 j) .. + 7, weight copy j rows 16 (w + 8 j) .. + 15; the swizzles do not depend on j.
+  uint32_t xoff[C::kXCopies], wsrc_off[C::kWCopies];
+  const char* xbase = static_cast<const char*>(p.x) + m0 * p.x_stride * 2;
+  const uint8_t* wbase = p.packed ? p.w + n0 / 16 * nkb * 2048 : p.w + n0 * p.K;
+#pragma unroll
+  for (int j = 0; j < C::kXCopies; ++j) {
+    const int row = 8 * (wave + 8 * j) + (lane >> 3);
+    xoff[j] = static_cast<uint32_t>(min64(row, p.M - 1 - m0) * p.x_stride * 2) + 16 * ((lane & 7) ^ ((row >> 1) & 7));
+  }
+#pragma unroll
+  for (int j = 0; j < C::kWCopies; ++j) {
+    const int reg = wave + 8 * j;  // 16 weight rows
+    const int row = 16 * reg + (lane >> 2);
+    // packed: lanes 0..31 the half's 512 contiguous bytes of 16-byte pieces h = 0 (see fp8_pack_kernel), lanes 32..63 of h = 1
+    wsrc_off[j] = p.packed ? static_cast<uint32_t>(min64(reg, (p.N - n0) / 16 - 1) * nkb * 2048) + 1024 * (lane >> 5) + 16 * (lane & 31)
+                         : static_cast<uint32_t>(min64(row, p.N - 1 - n0) * p.K) + 16 * ((lane & 3) ^ ((row >> 2) & 3));
+  }
+  const int64_t wblock = p.packed ? 2048 : KB;     // weight bytes from one block to the next, and
+  const int64_t whalf = p.packed ? 512 : C::SK;    // from its first half to its second
+  auto issue_copy = [&](int stage, int j) {  // copy j of a stage (past the last one: that one again)
+    const uint32_t base = smem_lds + static_cast<uint32_t>(stage % C::kStages) * C::kBuf;
+    const int64_t s = min(stage, ns - 1);
+    if (j < C::kXCopies)
+      lds_copy16_at(xbase + s * C::SK * 2, xoff[j], base + 1024u * static_cast<uint32_t>(wave + 8 * j));
+    else
+      lds_copy16_at(wbase + (s >> 1) * wblock + (s & 1) * whalf, wsrc_off[j - C::kXCopies],
+                    base + C::kXBytes + 1024u * static_cast<uint32_t>(wave + 8 * (j - C::kXCopies)));
+  };
+  // the block scales of the workgroup's weight rows (before the copies, so that waiting for them does not wait for
+  // those); the first barrier of the loop makes them visible
+  float* s_scale = reinterpret_cast<float*>(smem + C::kStages * C::kBuf);
+  for (int64_t i = tid; i < C::kScaleRows * nkb; i += 512) {
+    const int64_t row = min64(n0 / KB + i / nkb, p.N / KB - 1);
+    s_scale[i] = bf16_to_f32(p.scale[row * p.scale_cols + i % nkb]);
+  }
+#pragma unroll
+  for (int s = 0; s < C::kStages - 1; ++s)
+#pragma unroll
+    for (int j = 0; j < C::kCopies; ++j) issue_copy(s, j);
+
+  const int wm = wave % WM, wn = wave / WM;
+  const int l31 = lane & 31, h = lane >> 5;
+  const int xrow = 32 * MT * wm + l31;  // + 32 per x tile: the same (row / 2) mod 8
+  const int wrow = 32 * NT * wn + l31;  // + 32 per weight tile: the same (row / 4) mod 4
+  const unsigned char* xrd = smem + xrow * (C::SK * 2);
+  // this lane's weight pieces of step j: packed order or swizzled rows, 2 KB per 32 rows either way
+  int woff[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    woff[j] = C::kXBytes + (p.packed ? (wrow >> 4) * 1024 + 512 * h + 16 * (16 * j + (wrow & 15)) : wrow * C::SK + 16 * ((2 * j + h) ^ ((wrow >> 2) & 3)));
+  const int xsw = (xrow >> 1) & 7;
+  const float* sc_row = s_scale + (32 * NT * wn / KB) * nkb;
+  f32x16_v acc[MT][NT];
+  f32x16_v zero;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) zero[e] = 0.f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[i][n] = zero;
+
+  f32x16_v tmp[MT][NT];  // the block's sums, multiplied into acc before the next block's first products
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) tmp[i][n] = zero;
+  float sc = 0.f;
+  V w[NT][4], x[MT][4];
+  // k-step 2 j + e of a stage: lane half h holds columns 32 j + 16 h + 8 e .. + 7 of both operands
+  auto load_phase = [&](int s, bool first) {
+    const int buf = (s % C::kStages) * C::kBuf;
+    u32x4_v raw[NT][2];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) raw[n][j] = *reinterpret_cast<const u32x4_v*>(smem + buf + n * 32 * C::SK + woff[j]);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        x[i][q] = *reinterpret_cast<const V*>(xrd + buf + i * 32 * C::SK * 2 + 16 * ((4 * (q >> 1) + 2 * h + (q & 1)) ^ xsw));
+    __builtin_amdgcn_sched_barrier(0);  // reads first
+    if (first) {
+      acc[MT - 1][NT - 1] += sc * tmp[MT - 1][NT - 1];
+      sc = sc_row[s >> 1];
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        w[n][2 * j] = fp8x8_operand<V>(raw[n][j][0], raw[n][j][1]);
+        w[n][2 * j + 1] = fp8x8_operand<V>(raw[n][j][2], raw[n][j][3]);
+      }
+    // Copies in flight here: stages s + 1 and s + 2.  s + 1 has landed before the barrier that opens the first phase that
+    // reads it (the other waves' next one); s + 3 goes, in the product phase, to the buffer of s - 1, which both halves
+    // have read by then.
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(C::kCopies) : "memory");
+    phase_barrier();
+  };
+  // One output tile after the other; behind the second half's products of a tile the finished sums of the one before it
+  // go into acc between the MFMAs, four FMAs to one (an MFMA takes 32 cycles); the last tile's wait for the load phase
+  auto product_phase = [&](int s, bool first) {
+    __builtin_amdgcn_s_setprio(1);
+    constexpr int T = MT * NT;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int i = t / NT, n = t % NT;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        tmp[i][n] = mfma32(x[i][q], w[n][q], first && q == 0 ? zero : tmp[i][n]);
+        constexpr int per = 4 * T / C::kCopies;
+        if ((4 * t + q) % per == per - 1 && (4 * t + q) / per < C::kCopies) issue_copy(s + C::kStages - 1, (4 * t + q) / per);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!first && t > 0 && q > 0) {
+          const int pi = (t - 1) / NT, pn = (t - 1) % NT;
+#pragma unroll
+          for (int e = 16 * (q - 1) / 3; e < 16 * q / 3; ++e) acc[pi][pn][e] += sc * tmp[pi][pn][e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    phase_barrier();
+  };
+  // stage 0 has landed; from here waves 4..7 run one phase behind
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * C::kCopies) : "memory");
+  phase_barrier();
+  if (wave >= 4) phase_barrier();
+  for (int s = 0; s < ns; s += 2) {
+    load_phase(s, true);
+    product_phase(s, true);
+    load_phase(s + 1, false);
+    product_phase(s + 1, false);
+  }
+  if (wave < 4) phase_barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the last stage write LDS, too
+  acc[MT - 1][NT - 1] += sc * tmp[MT - 1][NT - 1];
+
+  // lane (h, l31), register e of tile (i, n): y[m0 + 32 (MT wm + i) + 8 (e / 4) + 4 h + e % 4][n0 + 32 (NT wn + n) + l31]
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int64_t col = n0 + 32 * (NT * wn + n) + l31;
+      if (col >= p.N) continue;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int64_t m = m0 + 32 * (MT * wm + i) + 8 * (e >> 2) + 4 * h + (e & 3);
+        if (m >= p.M) continue;
+        if (p.y_f32)
+          static_cast<float*>(p.y)[m * p.y_stride + col] = acc[i][n][e];
+        else
+          static_cast<bf16_t*>(p.y)[m * p.y_stride + col] = f32_to_bf16(acc[i][n][e]);
+      }
+    }
+}
+
 // fp32 x (16 rows or more) to fp16 once per call, round to nearest even (the reference's
 // float_rows_to_half_kernel, src/csrc/fp8_linear_cuda.cu:146-150): staging 16-bit x keeps the
 // main kernel's register ring small enough for its LDS operand reads to overlap.
@@ -678,7 +925,10 @@ __global__ __launch_bounds__(256) void fp8_cast_x_kernel(const float* __restrict
   *reinterpret_cast<f16x8_v*>(out + m * K + k) = r;
 }
 
+constexpr int64_t kBlockMaxStride = 1 << 23;  // elements: the block path's lane offsets (128 rows) stay below 2^31 bytes
+
 struct Plan {
+  int block;  // 16-bit x of more than 128 rows: the block kernel, 1 / 2 / 3 tiles of 128 x 256 / 128 x 128 / 64 x 128
   int xres;  // 16-bit x of 17..256 rows, in_features <= XR_KMAX: the x-resident kernel
   int wide;  // 16-bit x of 17..256 rows: the wide kernel (no K split), xt tiles of 16 rows
   int xt;
@@ -694,6 +944,27 @@ struct Plan {
 // workgroups with at least four K blocks each.
 inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
   Plan pl{};
+  // Block path: the largest tile that gives at least 192 of the 256 CUs a workgroup (160 for the smallest, whose
+  // workgroups are short), up to 128 rows the x-resident and wide kernels.  Both sides measured (us, fp32 x, packed):
+  // 128 x 256 against 128 x 128 at 192 tiles (768 x 8192 x 2048) 38.6 : 44.8, at 128 tiles (1024 x 4096 x 2048) 35.5 : 29.4;
+  // 128 x 128 against 64 x 128 at 192 tiles (768 x 4096 x 2048) 26.5 : 27.0, at 128 tiles (1024 x 2048 x 4096) 39.9 : 34.7;
+  // 64 x 128 against the paths below at 160 tiles (300 x 4096 x 2048) 19.2 : 27.2, at 128 tiles (512 x 2048 x 4096)
+  // 31.5 : 29.0 and (256 x 4096 x 2048) 19.0 : 14.2.
+  if (M > 128) {
+    const int64_t tm = (M + 127) / 128, tn = N / 128;
+    pl.block = tm * ((tn + 1) / 2) >= 192 ? 1 : tm * tn >= 192 ? 2 : (M + 63) / 64 * tn >= 160 ? 3 : 0;
+  }
+  if (pl.block) {
+    // bf16 rows too far apart for 32-bit offsets: the wide kernel
+    pl.wide = 1;
+    pl.xt = 4;
+    pl.mtiles = (M + 63) / 64;
+    pl.ntiles = N / WN;
+    pl.ksplit = 1;
+    pl.blocks_per_split = static_cast<int>(K / KB);
+    pl.workspace = M * K * 2;  // the fp16 copy of an fp32 x
+    return pl;
+  }
   if (M > 16 && M <= 256 && K <= XR_KMAX) {
     // x is 16-bit here in both input dtypes (fp32 x of 16 rows or more is cast to fp16 first)
     pl.xres = 1;
@@ -754,6 +1025,23 @@ int launch_xres(const Plan& pl, const Params& p, hipStream_t stream) {
   }
   const dim3 grid(static_cast<unsigned>(pl.ntiles), static_cast<unsigned>(pl.mtiles));
   hipLaunchKernelGGL((fp8_linear_xres_kernel<MODE, XCAST>), grid, dim3(WNT), kXresBytes, stream, p);
+  return 0;
+}
+
+template <int MODE, int MT, int NT, int WM, int WN>
+int launch_block(const Params& p, hipStream_t stream) {
+  using C = BlockCfg<MT, NT, WM, WN>;
+  static bool attr_set = false;  // the ring is above the 64 KB default of dynamic LDS
+  if (!attr_set) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fp8_linear_block_kernel<MODE, MT, NT, WM, WN>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, C::bytes(KB * MAX_KB));
+    if (err != hipSuccess) return fail("fp8_linear: cannot reserve %d bytes of LDS: %s", C::bytes(KB * MAX_KB), hipGetErrorString(err));
+    attr_set = true;
+  }
+  const int64_t tm = (p.M + C::TM - 1) / C::TM, tn = (p.N + C::TN - 1) / C::TN;
+  QA_REQUIRE(tm * tn <= 0x7ffffff0, "fp8_linear: shape too large");
+  hipLaunchKernelGGL((fp8_linear_block_kernel<MODE, MT, NT, WM, WN>), dim3(static_cast<unsigned>((tm * tn + 7) / 8 * 8)), dim3(512),
+                     static_cast<size_t>(C::bytes(p.K)), stream, p, static_cast<int>(tm), static_cast<int>(tn));
   return 0;
 }
 
@@ -853,6 +1141,18 @@ extern "C" int qa_fp8_linear(const void* x, int32_t x_dtype, int64_t x_stride, i
     {
       KernelTimer timer_("fp8_linear", stream);
       rc = xcast ? launch_xres<X_F16, true>(pl, p, stream) : launch_xres<X_BF16, false>(pl, p, stream);
+    }
+    if (rc) return rc;
+    return check_launch("fp8_linear");
+  }
+  if (pl.block && p.x_stride <= kBlockMaxStride) {
+    int rc = 0;
+    {
+      KernelTimer timer_("fp8_linear", stream);
+      if (mode == X_F16)
+        rc = pl.block == 1 ? launch_block<X_F16, 2, 2, 2, 4>(p, stream) : pl.block == 2 ? launch_block<X_F16, 1, 2, 4, 2>(p, stream) : launch_block<X_F16, 1, 1, 2, 4>(p, stream);
+      else
+        rc = pl.block == 1 ? launch_block<X_BF16, 2, 2, 2, 4>(p, stream) : pl.block == 2 ? launch_block<X_BF16, 1, 2, 4, 2>(p, stream) : launch_block<X_BF16, 1, 1, 2, 4>(p, stream);
     }
     if (rc) return rc;
     return check_launch("fp8_linear");
