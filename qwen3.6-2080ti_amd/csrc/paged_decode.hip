@@ -351,11 +351,13 @@ __global__ __launch_bounds__(256, QA_DECODE_WAVES_PER_SIMD) void decode_partial_
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t wid = static_cast<int64_t>(blockIdx.x) * kMfmaWaves + wave;
-  const int64_t W = p.n_waves;
   const int64_t T = uniform64(total_tiles(p, lane));
+  // With fewer tiles than waves launched (tables much wider than the contexts) only the first T waves
+  // work: the combine reads every slot from a row group's first wave to its last, so none may be idle.
+  const int64_t W = min64(p.n_waves, T);
+  if (wid >= W) return;
   const int64_t lo = T * wid / W;
   const int64_t hi = T * (wid + 1) / W;
-  if (lo >= hi) return;
   TileCursor cur = locate_tile(p, lo, lane);
   cur.b = __builtin_amdgcn_readfirstlane(cur.b);
   cur.g = __builtin_amdgcn_readfirstlane(cur.g);
