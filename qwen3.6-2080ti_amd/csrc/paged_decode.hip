@@ -212,6 +212,10 @@ constexpr int kVtPad = 16;            // 8-byte units of padding per token quad
 constexpr int kWaveGroup = QA_DECODE_GROUP;  // blocks per two-phase group
 constexpr int kMaxDecodeWaves = 1024 * QA_DECODE_WAVES_PER_SIMD;  // all resident at once on 256 CUs
 constexpr int kMinTilesPerWave = 8;
+// With few row groups the chip is not full and a wave's tiles are a chain of dependent loads, 1 to 2 us a
+// tile, so the launch is made of shorter chains: see decode_waves.
+constexpr int kFineTilesPerWave = 2;
+constexpr int64_t kFineRowGroups = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ __forceinline__ int vt_swizzle(int d) { return d ^ ((d >> 5) & 7); }
@@ -610,6 +614,83 @@ __global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_balanced(De
   for (int i = 0; i < CPL; ++i) Elem<QT>::store(out + i, o[i]);
 }
 
+// The same merge with kSplitCombineWaves waves per (row, head), for row groups of many partials: bound by
+// the latency of its loads, so each wave merges a contiguous share, kSplitCombineRows rows in flight at a
+// time (64 registers: 16 waves a workgroup leave 128), and the waves' (m, l, o) meet in LDS.
+constexpr int kSplitCombineWaves = 16;
+constexpr int kSplitCombineRows = 16;
+
+template <typename QT, int D>
+__global__ __launch_bounds__(64 * kSplitCombineWaves) void decode_combine_split(DecodeParams p) {
+  constexpr int CPL = D / 64;
+  typedef float vec_t __attribute__((ext_vector_type(CPL)));
+  __shared__ __align__(16) float part[kSplitCombineWaves][D];
+  __shared__ float part_m[kSplitCombineWaves], part_l[kSplitCombineWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bh = blockIdx.x;
+  const int b = bh / p.H;
+  const int h = bh - b * p.H;
+  const int g = h / p.G;
+  const int hh = h - g * p.G;
+  QT* out = reinterpret_cast<QT*>(p.out) + static_cast<int64_t>(bh) * D;
+
+  const int64_t rg = static_cast<int64_t>(b) * p.Hkv + g;
+  const int32_t w_first = p.rg_waves[2 * rg];
+  const int32_t w_last = p.rg_waves[2 * rg + 1];
+  if (row_tiles(p, b) == 0) {  // the whole workgroup: its row-group record is stale and not read
+    if (threadIdx.x < D) Elem<QT>::store(out + threadIdx.x, 0.f);
+    return;
+  }
+  const int n = w_last - w_first + 1;
+  const int64_t slot0 = w_first + rg;
+  const float* ml = p.part_ml + (slot0 * p.G + hh) * 2;
+  const float* po = p.part_o + (slot0 * p.G + hh) * D + CPL * lane;
+  const int64_t sml = 2 * static_cast<int64_t>(p.G);
+  const int64_t so = static_cast<int64_t>(p.G) * D;
+
+  const int end = n * (wave + 1) / kSplitCombineWaves;
+  float m_run = -INFINITY, den = 0.f;
+  vec_t acc = vec_t(0.f);
+  for (int c = n * wave / kSplitCombineWaves; c < end; c += kSplitCombineRows) {
+    const int cnt = min(kSplitCombineRows, end - c);
+    const float2 e = lane < cnt ? *reinterpret_cast<const float2*>(ml + (c + lane) * sml) : make_float2(-INFINITY, 0.f);
+    vec_t rows[kSplitCombineRows];
+#pragma unroll
+    for (int s = 0; s < kSplitCombineRows; ++s) rows[s] = s < cnt ? *reinterpret_cast<const vec_t*>(po + (c + s) * so) : vec_t(0.f);
+    const float m_new = fmaxf(m_run, wave_max(e.x));
+    const float use = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = exp2f(m_run - use);
+    m_run = m_new;
+    const float f = lane < cnt ? exp2f(e.x - use) : 0.f;
+    den = den * corr + f * e.y;
+    acc *= corr;
+#pragma unroll
+    for (int s = 0; s < kSplitCombineRows; ++s)
+      if (s < cnt) acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), s)) * rows[s];
+  }
+  den = wave_sum(den);
+  *reinterpret_cast<vec_t*>(&part[wave][CPL * lane]) = acc;
+  if (lane == 0) {
+    part_m[wave] = m_run;
+    part_l[wave] = den;
+  }
+  __syncthreads();
+  if (threadIdx.x >= D) return;
+  float big = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kSplitCombineWaves; ++w) big = fmaxf(big, part_m[w]);
+  const float use = big == -INFINITY ? 0.f : big;
+  float l = 0.f, o = 0.f;
+#pragma unroll
+  for (int w = 0; w < kSplitCombineWaves; ++w) {
+    const float f = exp2f(part_m[w] - use);
+    l += f * part_l[w];
+    o += f * part[w][threadIdx.x];
+  }
+  Elem<QT>::store(out + threadIdx.x, l > 0.f ? o / l : 0.f);
+}
+
 // Merge the splits of one (row, head): O = sum_s e^{m_s-M} o_s / sum_s e^{m_s-M} l_s.
 // Rows without any visible token (length <= 0, or only invalid blocks) get 0.
 // Split weights are computed once per split into LDS; each thread then owns
@@ -682,23 +763,42 @@ static int choose_split_tokens(int64_t max_tokens, int block_size) {
 }
 
 // Waves of the balanced MFMA schedule for `row_groups` rows of up to max_tokens
-// tokens: at least kMinTilesPerWave tiles each when every row is full, at most
+// tokens: at least min_tiles tiles each when every row is full, at most
 // kMaxDecodeWaves, a whole number of 4-wave workgroups.
-static int64_t balanced_waves(int64_t row_groups, int64_t max_tokens) {
+static int64_t balanced_waves(int64_t row_groups, int64_t max_tokens, int min_tiles) {
   const int64_t tiles = row_groups * ceil_div(std::max<int64_t>(max_tokens, 1), 16);
-  const int64_t wgs = std::min<int64_t>(kMaxDecodeWaves / kMfmaWaves, std::max<int64_t>(1, ceil_div(tiles, kMfmaWaves * kMinTilesPerWave)));
+  const int64_t wgs = std::min<int64_t>(kMaxDecodeWaves / kMfmaWaves, std::max<int64_t>(1, ceil_div(tiles, kMfmaWaves * min_tiles)));
   return wgs * kMfmaWaves;
 }
+
+// Waves of a launch.  Up to kFineRowGroups row groups: chains of kFineTilesPerWave tiles where that still
+// leaves the merge few partials, which is 512 a row group with decode_combine_split (up to 16 row groups)
+// and 16 with decode_combine_balanced.  Measured, 16 heads on 2 x 256 (8 tiles a wave before -> now, us):
+// 4 rows of 512 tokens 23.9 -> 15.7; 1 row of 8192 27.5 -> 19.5 (1 tile a wave 23.1: the merge), of 32768
+// 47.3 -> 27.2; 16 rows of 100 to 2048 tokens stay at 23 (32 partials a row group 24.9).  More row groups
+// fill the chip with kMinTilesPerWave (64 rows of 100 to 600 tokens: 23.0 and 22.9).
+static int64_t decode_waves(int64_t row_groups, int64_t max_tokens) {
+  const int64_t coarse = balanced_waves(row_groups, max_tokens, kMinTilesPerWave);
+  if (row_groups > kFineRowGroups) return coarse;
+  const int64_t cap = row_groups <= 16 ? 512 * row_groups : 16 * row_groups;  // multiples of kMfmaWaves
+  return std::max(coarse, std::min(cap, balanced_waves(row_groups, max_tokens, kFineTilesPerWave)));
+}
+
+// Which merge: from a mean of 32 partials a row group, as many as a wave of decode_combine_balanced has
+// in flight, the workgroup of decode_combine_split (4 rows of 100 to 8192 tokens 24.4 against 45.3 us, 8
+// of 700 to 4096 with D 128 17.7 against 21.7); below, its barrier and its 16 waves a head cost more than
+// they save (4 rows of 512, 16 partials: 17.2 against 15.7; 32 rows of 100 to 2048: 30.9 against 26.3).
+static bool split_combine(const DecodeParams& p) { return p.n_waves >= 32 * static_cast<int64_t>(p.B) * p.Hkv; }
 
 // Bytes of workspace either path may need.  The generic path stores
 // (B*H, n_splits, D + 2) floats; the MFMA path (W + B*H_kv) slots of G heads
 // plus two int32 per row group, bounded here with H_kv <= H and W computed
-// for H row groups per row.
+// for H row groups per row and the shortest chains.
 static int64_t decode_workspace_bytes(int64_t batch, int heads, int head_dim, int64_t max_tokens, int block_size) {
   const int split = choose_split_tokens(max_tokens, block_size);
   const int64_t n_splits = std::max<int64_t>(1, ceil_div(std::max<int64_t>(max_tokens, 1), split));
   const int64_t generic = batch * heads * n_splits * (head_dim + 2);
-  const int64_t balanced = (balanced_waves(batch * heads, max_tokens) + batch) * heads * (head_dim + 2) + 2 * batch * heads;
+  const int64_t balanced = (balanced_waves(batch * heads, max_tokens, kFineTilesPerWave) + batch) * heads * (head_dim + 2) + 2 * batch * heads;
   return std::max(generic, balanced) * static_cast<int64_t>(sizeof(float));
 }
 
@@ -744,7 +844,10 @@ static int launch_mfma_d(DecodeParams& p, hipStream_t stream) {
   if (int rc = check_launch("decode_partial_mfma")) return rc;
   {
     KernelTimer timer_("decode_combine", stream);
-    hipLaunchKernelGGL((decode_combine_balanced<bf16_t, D>), dim3(ceil_div(p.B * p.H, kCombineWaves)), dim3(64 * kCombineWaves), 0, stream, p);
+    if (split_combine(p))
+      hipLaunchKernelGGL((decode_combine_split<bf16_t, D>), dim3(p.B * p.H), dim3(64 * kSplitCombineWaves), 0, stream, p);
+    else
+      hipLaunchKernelGGL((decode_combine_balanced<bf16_t, D>), dim3(ceil_div(p.B * p.H, kCombineWaves)), dim3(64 * kCombineWaves), 0, stream, p);
   }
   return check_launch("decode_combine");
 }
@@ -847,7 +950,7 @@ static int run_decode(const DecodeHostArgs& a, hipStream_t stream) {
   p.split_tokens = choose_split_tokens(a.max_tokens, a.block_size);
   p.n_splits = static_cast<int>(std::max<int64_t>(1, ceil_div(std::max<int64_t>(a.max_tokens, 1), p.split_tokens)));
   QA_REQUIRE(p.n_splits <= kCombineMaxSplits, "paged decode: %lld tokens need more than %d splits", static_cast<long long>(a.max_tokens), kCombineMaxSplits);
-  p.n_waves = static_cast<int>(balanced_waves(static_cast<int64_t>(p.B) * p.Hkv, a.max_tokens));
+  p.n_waves = static_cast<int>(decode_waves(static_cast<int64_t>(p.B) * p.Hkv, a.max_tokens));
   const bool mfma = a.q_dtype == QA_BF16 && kv.dtype == QA_BF16 && mfma_eligible(p, a, kv);
   // bytes of the path taken (qa_paged_attention_decode_workspace returns the larger of the two)
   const int64_t slots = static_cast<int64_t>(p.n_waves) + static_cast<int64_t>(p.B) * p.Hkv;

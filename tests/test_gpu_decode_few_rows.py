@@ -1,6 +1,7 @@
-"""Batched decode with tables wider than the contexts against the CPU oracle.
+"""Batched decode with few row groups against the CPU oracle: short chains, both merges, tables wider than the contexts.
 
-Tolerance for bf16 outputs as in the other decode tests: ``atol = rtol = 2e-2``.
+The launch has ``min(1024, tiles / 2)`` waves for up to 64 row groups, and the merge takes a workgroup per head
+from 32 partials a row group.  Tolerance for bf16 outputs as in the other decode tests: ``atol = rtol = 2e-2``.
 """
 
 from __future__ import annotations
@@ -35,9 +36,17 @@ def _case(lens, heads, kv_heads, dim, width, index, seed):
 @pytest.mark.parametrize(
     "lens, heads, kv_heads, dim, width, index",
     [
+        ([1], 16, 2, 256, 1, torch.int32),  # one tile, one wave per row group
+        ([17], 16, 1, 128, 2, torch.int64),
         ([40], 16, 2, 256, 2048, torch.int32),  # table far wider than the context: most launched waves idle
         ([5, 0, 33, 1], 16, 2, 256, 512, torch.int32),  # the same with an empty row, workgroup merge
         ([0, 0], 8, 2, 128, 64, torch.int32),  # nothing to attend to at all
+        ([512] * 4, 16, 2, 256, 0, torch.int32),  # 16 partials a row group: wave merge
+        ([1023], 16, 2, 256, 0, torch.int32),  # 32 partials: workgroup merge
+        ([8191], 16, 1, 128, 0, torch.int32),  # 256 partials, one row group
+        ([4000, 1, 15, 16, 2047], 8, 2, 128, 0, torch.int64),  # skewed rows
+        ([300 + 7 * r for r in range(17)], 8, 2, 128, 0, torch.int32),  # 34 row groups
+        ([200 + 3 * r for r in range(33)], 4, 2, 128, 0, torch.int32),  # 66 row groups: past the rule
     ],
 )
 def test_few_rows_match_oracle(lens, heads, kv_heads, dim, width, index) -> None:
