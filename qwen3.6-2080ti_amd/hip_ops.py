@@ -36,6 +36,10 @@ _DTYPE_CODES = {
 }
 
 
+_FLOAT_DTYPES = (torch.float32, torch.bfloat16)
+_INDEX_DTYPES = (torch.int32, torch.int64)
+
+
 def _code(tensor: torch.Tensor) -> int:
     try:
         return _DTYPE_CODES[tensor.dtype]
@@ -43,12 +47,23 @@ def _code(tensor: torch.Tensor) -> int:
         raise RuntimeError(f"unsupported dtype {tensor.dtype}") from exc
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# The smallest calls are bound by this file and not by their kernels, so what every call runs stays lean: the
+# raw stream handle without a Stream object, pointers as plain integers, no message formatted before a check fails.
+def _stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
-def _ptr(tensor: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if tensor is None else tensor.data_ptr())
+def _ptr(tensor: torch.Tensor | None) -> int:
+    return 0 if tensor is None else tensor.data_ptr()
+
+
+def _flat(tensor: torch.Tensor) -> torch.Tensor:
+    return tensor if tensor.dim() == 1 else tensor.reshape(-1)
+
+
+def _vector_on(tensor: torch.Tensor, device: torch.device) -> torch.Tensor:
+    flat = _flat(tensor)
+    return (flat if flat.device == device else flat.to(device=device)).contiguous()
 
 
 def _require(cond: bool, message: str) -> None:
@@ -57,17 +72,20 @@ def _require(cond: bool, message: str) -> None:
 
 
 def _require_cuda(tensor: Any, name: str, device: torch.device | None = None) -> None:
-    _require(isinstance(tensor, torch.Tensor) and tensor.is_cuda, f"{name} must be CUDA")
-    if device is not None:
-        _require(tensor.device == device, f"{name} must be on same CUDA device as query")
+    if not (isinstance(tensor, torch.Tensor) and tensor.is_cuda):
+        raise RuntimeError(f"{name} must be CUDA")
+    if device is not None and tensor.device != device:
+        raise RuntimeError(f"{name} must be on same CUDA device as query")
 
 
 def _float_dtype(tensor: torch.Tensor, name: str) -> None:
-    _require(tensor.dtype in (torch.float32, torch.bfloat16), f"{name} must be float32 or bfloat16")
+    if tensor.dtype not in _FLOAT_DTYPES:
+        raise RuntimeError(f"{name} must be float32 or bfloat16")
 
 
 def _index_dtype(tensor: torch.Tensor, name: str) -> None:
-    _require(tensor.dtype in (torch.int32, torch.int64), f"{name} must be int64/torch.long or int32")
+    if tensor.dtype not in _INDEX_DTYPES:
+        raise RuntimeError(f"{name} must be int64/torch.long or int32")
 
 
 def _pool_descriptor(key_pool: torch.Tensor, value_pool: torch.Tensor, layout: str) -> L.PagedKV:
@@ -76,28 +94,16 @@ def _pool_descriptor(key_pool: torch.Tensor, value_pool: torch.Tensor, layout: s
     _require(key_pool.dtype == value_pool.dtype, "key/value blocks must have the same dtype")
     _require(key_pool.stride(-1) == 1 and value_pool.stride(-1) == 1, "key/value blocks must be contiguous in head_dim")
     _require(key_pool.stride() == value_pool.stride(), "key/value blocks must share strides")
-    desc = L.PagedKV()
-    desc.key = key_pool.data_ptr()
-    desc.value = value_pool.data_ptr()
-    desc.row_key_ptrs = None
-    desc.row_value_ptrs = None
-    desc.row_blocks = None
-    desc.dtype = _code(key_pool)
+    shape, strides = key_pool.shape, key_pool.stride()
     if layout == "reference":  # (B, heads, P, bs, D)
-        desc.num_blocks = key_pool.shape[2]
-        desc.stride_batch = key_pool.stride(0)
-        desc.stride_head = key_pool.stride(1)
-        desc.stride_block = key_pool.stride(2)
-        desc.stride_token = key_pool.stride(3)
-        desc.kv_heads = key_pool.shape[1]
+        heads, blocks = shape[1], shape[2]
+        stride_batch, stride_head, stride_block, stride_token = strides[:4]
     else:  # shared (P, H_kv, bs, D)
-        desc.num_blocks = key_pool.shape[0]
-        desc.stride_batch = 0
-        desc.stride_block = key_pool.stride(0)
-        desc.stride_head = key_pool.stride(1)
-        desc.stride_token = key_pool.stride(2)
-        desc.kv_heads = key_pool.shape[1]
-    return desc
+        blocks, heads = shape[0], shape[1]
+        stride_batch = 0
+        stride_block, stride_head, stride_token = strides[:3]
+    return L.PagedKV(key_pool.data_ptr(), value_pool.data_ptr(), None, None, None, blocks, stride_batch, stride_block, stride_head,
+                     stride_token, heads, _code(key_pool))
 
 
 def _decode_workspace(lib: Any, batch: int, heads: int, head_dim: int, max_tokens: int, block_size: int, device: torch.device) -> torch.Tensor:
@@ -360,7 +366,7 @@ def paged_kv_append(
     tables = block_tables.contiguous()
     table_stride = tables.stride(0) if tables.dim() == 2 else 0
     max_blocks = tables.shape[-1]
-    start_ptr, start_code, start_scalar = ctypes.c_void_p(0), L.QA_I64, 0
+    start_ptr, start_code, start_scalar = 0, L.QA_I64, 0
     if isinstance(starts, torch.Tensor):
         _require_cuda(starts, "starts", device)
         _index_dtype(starts, "starts")
@@ -368,7 +374,7 @@ def paged_kv_append(
         start_ptr, start_code = _ptr(starts), _code(starts)
     else:
         start_scalar = int(starts)
-    count_ptr, count_code = ctypes.c_void_p(0), L.QA_I64
+    count_ptr, count_code = 0, L.QA_I64
     if counts is not None:
         _require_cuda(counts, "counts", device)
         _index_dtype(counts, "counts")
@@ -417,7 +423,7 @@ def paged_kv_reserve(
     _require(free_list.dtype == torch.int32 and free_list.dim() == 1 and free_list.is_contiguous(), "free_list must be a contiguous int32 vector")
     _require(free_state.dtype == torch.int32 and free_state.numel() == 2 and free_state.is_contiguous(), "free_state must be int32 [head, count]")
     _require(status.dtype == torch.int32 and status.numel() >= 1, "status must be an int32 tensor")
-    count_ptr, count_code, count_scalar = ctypes.c_void_p(0), L.QA_I64, 0
+    count_ptr, count_code, count_scalar = 0, L.QA_I64, 0
     if isinstance(counts, torch.Tensor):
         _require_cuda(counts, "counts", device)
         _index_dtype(counts, "counts")
@@ -426,7 +432,7 @@ def paged_kv_reserve(
     else:
         count_scalar = int(counts)
         _require(count_scalar >= 0, "counts must be non-negative")
-    pos_ptr, pos_code = ctypes.c_void_p(0), L.QA_I64
+    pos_ptr, pos_code = 0, L.QA_I64
     if positions is not None:
         _require_cuda(positions, "positions", device)
         _index_dtype(positions, "positions")
@@ -491,8 +497,10 @@ def fp8_e4m3_bf16_linear(input: torch.Tensor, weight: torch.Tensor | PackedFp8We
     _require(input.shape[-1] == cols, "input last dim must match weight cols")
     _require(rows % 128 == 0, "weight rows must be divisible by 128 for the FP8 op")
     _require(cols % 128 == 0, "weight cols must be divisible by 128 for the FP8 op")
-    _require(tuple(scale.shape) == (rows // 128, cols // 128), "scale blocks mismatch")
-    x = input.contiguous().view(-1, cols)
+    _require(scale.shape == (rows // 128, cols // 128), "scale blocks mismatch")
+    x = input.contiguous()
+    if x.dim() != 2:
+        x = x.view(-1, cols)
     w = weight.data if packed else weight.contiguous()
     s = scale.contiguous()
     out = torch.empty((x.shape[0], rows), dtype=out_dtype, device=device)
@@ -503,7 +511,7 @@ def fp8_e4m3_bf16_linear(input: torch.Tensor, weight: torch.Tensor | PackedFp8We
         ws.numel(), _stream(device),
     )
     L.check(lib, status, "fp8_e4m3_bf16_linear")
-    return out.view(*input.shape[:-1], rows)
+    return out if input.dim() == 2 else out.view(*input.shape[:-1], rows)
 
 
 def paged_kv_gather(key_pool: torch.Tensor, value_pool: torch.Tensor, block_tables: torch.Tensor, valid: int, block_size: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -585,7 +593,9 @@ def linear_attention_recurrent_core(query: torch.Tensor, key: torch.Tensor, valu
 
 def _conv_weight(weight: torch.Tensor, channels: int, device: torch.device) -> torch.Tensor:
     _require_cuda(weight, "conv weight", device)
-    w = weight.reshape(weight.shape[0], weight.shape[-1]).float().contiguous()
+    w = weight if weight.dim() == 2 else weight.reshape(weight.shape[0], weight.shape[-1])
+    if w.dtype != torch.float32 or not w.is_contiguous():
+        w = w.float().contiguous()
     _require(w.shape[0] == channels, "conv weight must have one row per channel")
     return w
 
@@ -614,7 +624,7 @@ def causal_conv1d_prefill(
     new_state = torch.empty((batch, channels, kernel - 1), dtype=torch.float32, device=device)
     out = torch.empty((batch, seq, channels), dtype=out_dtype, device=device)
     status = lib.qa_causal_conv1d_prefill(
-        _ptr(x), _code(x), x.stride(0), x.stride(1), _ptr(state_in), _ptr(new_state), channels * (kernel - 1), ctypes.c_void_p(0), L.QA_I32,
+        _ptr(x), _code(x), x.stride(0), x.stride(1), _ptr(state_in), _ptr(new_state), channels * (kernel - 1), 0, L.QA_I32,
         batch, _ptr(w), batch, seq, channels, kernel, _ptr(out), _code(out), out.stride(0), out.stride(1), int(apply_silu), _stream(device),
     )
     L.check(lib, status, "causal_conv1d_prefill")
@@ -637,7 +647,7 @@ def causal_conv1d_update(x: torch.Tensor, conv_state: torch.Tensor, weight: torc
     _require_cuda(conv_state, "conv_state", device)
     _require(conv_state.dtype == torch.float32 and conv_state.is_contiguous(), "conv_state must be contiguous float32")
     _require(tuple(conv_state.shape[1:]) == (channels, kernel - 1), "conv_state must be (rows, channels, kernel-1)")
-    slot_ptr, slot_code = ctypes.c_void_p(0), L.QA_I32
+    slot_ptr, slot_code = 0, L.QA_I32
     if slots is not None:
         _require_cuda(slots, "slots", device)
         _index_dtype(slots, "slots")
@@ -692,9 +702,9 @@ def gated_delta_step(
     _require(a.shape == (batch, value_heads) and b.shape == (batch, value_heads), "a/b must be (batch, value_heads)")
     _require(a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16), "a/b must share a float32/bfloat16 dtype")
     a_c, b_c = a.contiguous(), b.contiguous()
-    alog = _f32_contig(a_log.reshape(-1), "a_log", device)
-    dtb = _f32_contig(dt_bias.reshape(-1), "dt_bias", device)
-    slot_ptr, slot_code = ctypes.c_void_p(0), L.QA_I32
+    alog = _f32_contig(_flat(a_log), "a_log", device)
+    dtb = _f32_contig(_flat(dt_bias), "dt_bias", device)
+    slot_ptr, slot_code = 0, L.QA_I32
     if slots is not None:
         _require_cuda(slots, "slots", device)
         _index_dtype(slots, "slots")
@@ -711,9 +721,9 @@ def gated_delta_step(
         _require_cuda(z, "z", device)
         _float_dtype(z, "z")
         _require(norm_weight is not None, "the output stage needs norm_weight")
-        zz = z.reshape(batch, value_heads * value_dim)
+        zz = z if z.shape == (batch, value_heads * value_dim) else z.reshape(batch, value_heads * value_dim)
         _require(zz.stride(-1) == 1, "z rows must be contiguous")
-        w = norm_weight.reshape(-1).to(device=device).contiguous()
+        w = _vector_on(norm_weight, device)
         _float_dtype(w, "norm_weight")
         _require(w.numel() == value_dim, "norm_weight must have value_dim elements")
         status = lib.qa_gated_delta_step_norm(
@@ -771,22 +781,22 @@ def gated_delta_step_conv(
     _require(a.shape == (batch, value_heads) and b.shape == (batch, value_heads), "a/b must be (batch, value_heads)")
     _require(a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16), "a/b must share a float32/bfloat16 dtype")
     a_c, b_c = a.contiguous(), b.contiguous()
-    alog = _f32_contig(a_log.reshape(-1), "a_log", device)
-    dtb = _f32_contig(dt_bias.reshape(-1), "dt_bias", device)
-    slot_ptr, slot_code = ctypes.c_void_p(0), L.QA_I32
+    alog = _f32_contig(_flat(a_log), "a_log", device)
+    dtb = _f32_contig(_flat(dt_bias), "dt_bias", device)
+    slot_ptr, slot_code = 0, L.QA_I32
     if slots is not None:
         _require_cuda(slots, "slots", device)
         _index_dtype(slots, "slots")
         slots = slots.contiguous()
         slot_ptr, slot_code = _ptr(slots), _code(slots)
-    z_ptr, z_code, z_sb, w_ptr, w_code = ctypes.c_void_p(0), L.QA_F32, 0, ctypes.c_void_p(0), L.QA_F32
+    z_ptr, z_code, z_sb, w_ptr, w_code = 0, L.QA_F32, 0, 0, L.QA_F32
     if z is not None:
         _require_cuda(z, "z", device)
         _float_dtype(z, "z")
         _require(norm_weight is not None, "the output stage needs norm_weight")
-        zz = z.reshape(batch, value_heads * value_dim)
+        zz = z if z.shape == (batch, value_heads * value_dim) else z.reshape(batch, value_heads * value_dim)
         _require(zz.stride(-1) == 1, "z rows must be contiguous")
-        nw = norm_weight.reshape(-1).to(device=device).contiguous()
+        nw = _vector_on(norm_weight, device)
         _float_dtype(nw, "norm_weight")
         _require(nw.numel() == value_dim, "norm_weight must have value_dim elements")
         z_ptr, z_code, z_sb, w_ptr, w_code = _ptr(zz), _code(zz), zz.stride(0), _ptr(nw), _code(nw)
@@ -839,8 +849,8 @@ def chunk_gated_delta_rule(
     _require(a.shape == (batch, seq, value_heads) and b.shape == a.shape, "a/b must be (batch, seq, value_heads)")
     _require(a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16), "a/b must share a float32/bfloat16 dtype")
     _require(a.stride() == b.stride() and a.stride(-1) == 1, "a/b must share strides with contiguous heads")
-    alog = _f32_contig(a_log.reshape(-1), "a_log", device)
-    dtb = _f32_contig(dt_bias.reshape(-1), "dt_bias", device)
+    alog = _f32_contig(_flat(a_log), "a_log", device)
+    dtb = _f32_contig(_flat(dt_bias), "dt_bias", device)
     w = _conv_weight(conv_weight, channels, device)
     _require(w.shape[1] == 4, "conv kernel must be 4")
     conv_in = None
@@ -886,7 +896,7 @@ def gated_rms_norm(core: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, ep
     x = core.reshape(-1, heads, head_dim)
     gate = z.reshape(*lead, heads, head_dim).reshape(-1, heads, head_dim)
     _require(gate.stride(-1) == 1, "z must have a contiguous head_dim axis")
-    w = weight.reshape(-1).to(device=device).contiguous()
+    w = _vector_on(weight, device)
     _float_dtype(w, "weight")
     _require(w.numel() == head_dim, "weight must have head_dim elements")
     out = torch.empty((x.shape[0], heads, head_dim), dtype=out_dtype or core.dtype, device=device)
@@ -960,14 +970,14 @@ def paged_attention_prefill(
     return out
 
 
-_INV_FREQ: dict[tuple[int, float, str], torch.Tensor] = {}
+_INV_FREQ: dict[tuple[int, float, torch.device], torch.Tensor] = {}
 
 
 def rope_inv_freq(rotary_dim: int, rope_theta: float, device: torch.device) -> torch.Tensor:
     """``inv_freq`` of ``rotary_embeddings`` (``src/reference_ops.py:203-213``), computed as the
     reference computes it (fp32 torch on the CPU), moved to ``device`` once per
     (rotary_dim, theta, device)."""
-    key = (int(rotary_dim), float(rope_theta), str(device))
+    key = (int(rotary_dim), float(rope_theta), device)
     cached = _INV_FREQ.get(key)
     if cached is None:
         inv = 1.0 / (float(rope_theta) ** (torch.arange(0, rotary_dim, 2, dtype=torch.float32) / rotary_dim))
@@ -976,7 +986,7 @@ def rope_inv_freq(rotary_dim: int, rope_theta: float, device: torch.device) -> t
     return cached
 
 
-_COS_SIN: dict[tuple[int, float, str], torch.Tensor] = {}
+_COS_SIN: dict[tuple[int, float, torch.device], torch.Tensor] = {}
 
 
 def rope_cos_sin_table(rotary_dim: int, rope_theta: float, positions: int, device: torch.device) -> torch.Tensor:
@@ -984,7 +994,7 @@ def rope_cos_sin_table(rotary_dim: int, rope_theta: float, positions: int, devic
     torch CPU operations of ``rotary_embeddings`` (``src/reference_ops.py:203-213``: fp32 angles,
     fp32 cos/sin, cast to bf16) so the values are the reference's bit for bit; cached per
     (rotary_dim, theta, device) and regrown when more positions are asked for."""
-    key = (int(rotary_dim), float(rope_theta), str(device))
+    key = (int(rotary_dim), float(rope_theta), device)
     cached = _COS_SIN.get(key)
     if cached is None or cached.shape[0] < positions:
         freqs = torch.outer(torch.arange(positions, dtype=torch.float32), rope_inv_freq(rotary_dim, rope_theta, torch.device("cpu")))
@@ -1044,7 +1054,8 @@ def qk_norm_rope_kv_append(
     _require(q3.dim() == 3 and q3.shape[2] == 2 * head_dim, "q_proj must be (tokens, heads, 2*head_dim)")
     _require(k3.shape == (tokens, kv_heads, head_dim) and v3.shape == (tokens, kv_heads, head_dim), "k_proj/v_proj must be (tokens, kv_heads, head_dim)")
     for tensor, name in ((q3, "q_proj"), (k3, "k_proj"), (v3, "v_proj"), (key_pool, "key_pool")):
-        _require(tensor.dtype == torch.bfloat16 and tensor.stride(-1) == 1, f"{name} must be bfloat16 with a contiguous last dimension")
+        if tensor.dtype != torch.bfloat16 or tensor.stride(-1) != 1:
+            raise RuntimeError(f"{name} must be bfloat16 with a contiguous last dimension")
     _float_dtype(q_norm_weight, "q_norm_weight")
     _require(q_norm_weight.dtype == k_norm_weight.dtype and q_norm_weight.shape == (head_dim,) and k_norm_weight.shape == (head_dim,),
              "norm weights must be (head_dim,) of one dtype")
@@ -1069,4 +1080,4 @@ def qk_norm_rope_kv_append(
         tables.shape[1], int(block_size), _ptr(query), _stream(device),
     )
     L.check(lib, status, "qk_norm_rope_kv_append")
-    return query, q3[..., head_dim:]
+    return query, q3.narrow(2, head_dim, head_dim)
