@@ -69,6 +69,7 @@ struct Params {
   int64_t table_stride, max_blocks;
   const bf16_t* gate;          // (token, H*D) or null
   int64_t gate_st, gate_sh;
+  int gate_vec;                // gate rows of every (token, head) are 8-byte aligned
   bf16_t* out;                 // (token, H, D) contiguous
   int64_t B;
   int H, Hkv, G, D;
@@ -561,6 +562,24 @@ __global__ __launch_bounds__(64 * (HMAX / HPW)) void prefill_kernel(Params p) {
     const float inv = l_part[hh] > 0.f ? 1.f / l_part[hh] : 0.f;
     bf16_t* orow = p.out + (tok * p.H + h) * static_cast<int64_t>(D);
     const bf16_t* grow = p.gate != nullptr ? p.gate + tok * p.gate_st + static_cast<int64_t>(h) * p.gate_sh : nullptr;
+    // The head's gate row, all loads in flight before any is used: fetched 2 bytes at a time inside the loop
+    // below, each dim tile waited for its own and a workgroup spent 12 us here (one row of 16 new tokens:
+    // 24.4 us, 12.4 without a gate; with the loads together 15.8).
+    uint2 graw[MT];
+    if (grow != nullptr) {
+      if (p.gate_vec) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) graw[t] = *reinterpret_cast<const uint2*>(grow + 16 * t + 4 * quad);
+      } else {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const bf16_t* e = grow + 16 * t + 4 * quad;
+          graw[t] = make_uint2(static_cast<uint32_t>(e[0]) | static_cast<uint32_t>(e[1]) << 16,
+                               static_cast<uint32_t>(e[2]) | static_cast<uint32_t>(e[3]) << 16);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // keeps the loads together
+    }
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const int d0 = 16 * t + 4 * quad;
@@ -568,7 +587,10 @@ __global__ __launch_bounds__(64 * (HMAX / HPW)) void prefill_kernel(Params p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         v[r] = o[hh][t][r] * inv;
-        if (grow != nullptr) v[r] *= 1.f / (1.f + __expf(-bf16_to_f32(grow[d0 + r])));
+        if (grow != nullptr) {
+          const uint32_t pair = r < 2 ? graw[t].x : graw[t].y;
+          v[r] *= 1.f / (1.f + __expf(-bf16_to_f32(static_cast<bf16_t>(r & 1 ? pair >> 16 : pair & 0xffffu))));
+        }
       }
       uint2 packed;
       packed.x = static_cast<uint32_t>(f32_to_bf16(v[0])) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16);
@@ -651,6 +673,7 @@ extern "C" int qa_paged_attention_prefill(const void* query, int32_t q_dtype, in
   p.gate = reinterpret_cast<const bf16_t*>(gate);
   p.gate_st = gate_stride_t;
   p.gate_sh = gate_stride_h != 0 ? gate_stride_h : head_dim;
+  p.gate_vec = (reinterpret_cast<uintptr_t>(gate) & 7u) == 0 && p.gate_st % 4 == 0 && p.gate_sh % 4 == 0;
   p.out = reinterpret_cast<bf16_t*>(output);
   p.B = batch;
   p.H = heads;
