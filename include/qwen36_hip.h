@@ -361,8 +361,10 @@ int qa_gated_delta_step_conv(const void* x, int32_t x_dtype, int64_t x_stride_b,
  * raw in_proj outputs.  mixed_qkv (B, T, 2*Hqk*dk + Hv*dv) bfloat16,
  * a, b (B, T, Hv), a_log/dt_bias (Hv) fp32, conv_weight (C, 4) fp32,
  * conv_state_in/out (B, C, 3) fp32 (NULL in = zeros, NULL out = not kept),
- * initial_state/final_state (B, Hv, dk, dv) fp32 (NULL in = zeros).  Writes
- * out (B, T, Hv, dv) float32/bfloat16.  Computes the conv1d + SiLU, L2 norm,
+ * initial_state/final_state (B, Hv, dk, dv) fp32 (NULL in = zeros).
+ * final_state may be initial_state; conv_state_out may be conv_state_in only
+ * for T <= 33, beyond that waves that nothing orders read the one and write
+ * the other.  Writes out (B, T, Hv, dv) float32/bfloat16.  Computes the conv1d + SiLU, L2 norm,
  * q scale and gating of src/reference_ops.py:240-283 and the recurrence of
  * :291-322 in 64-token chunks (WY/UT form) on fp16 MFMA with fp32
  * accumulation and an fp32 state.  dk = dv = 128, conv kernel 4.  The

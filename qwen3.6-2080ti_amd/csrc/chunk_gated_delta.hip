@@ -1484,20 +1484,6 @@ __global__ __launch_bounds__(256, 4) void blocks_kernel(BlocksParams bp) {
       if (kind == 1) *reinterpret_cast<f16x8_v*>(dst + j * DK) = o;
     }
   }
-  // conv state of the head's q and k channels: the raw inputs of the last three tokens
-  if (p.conv_out != nullptr && c == p.nch - 1) {
-    const int64_t ch = static_cast<int64_t>((tid < DK ? 0 : p.Hk) + hk) * DK + (tid & (DK - 1));
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      const int64_t t = p.T - 3 + s;
-      float val = 0.f;
-      if (t >= 0)
-        val = bf16_to_f32(p.x[b * p.x_sb + t * p.x_st + ch]);
-      else if (p.conv_in != nullptr)
-        val = p.conv_in[(b * p.C + ch) * (KCONV - 1) + (KCONV - 1) + t];
-      p.conv_out[(b * p.C + ch) * (KCONV - 1) + s] = val;
-    }
-  }
 
   const int64_t rec_step = p.nch * REC_BYTES;  // from one value head to the next
   unsigned char* rec_hk = bp.rec + ((b * p.Hv + static_cast<int64_t>(hk) * R) * p.nch + c) * REC_BYTES;
@@ -1535,6 +1521,21 @@ __global__ __launch_bounds__(256, 4) void blocks_kernel(BlocksParams bp) {
   };
   if (wave < R) gate(wave);
   lds_barrier();
+  // conv state of the head's q and k channels: the raw inputs of the last three tokens.  Behind the barrier: where
+  // conv_out is conv_in, a sequence of one chunk reads the old state above in other waves than write the new one here.
+  if (p.conv_out != nullptr && c == p.nch - 1) {
+    const int64_t ch = static_cast<int64_t>((tid < DK ? 0 : p.Hk) + hk) * DK + (tid & (DK - 1));
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const int64_t t = p.T - 3 + s;
+      float val = 0.f;
+      if (t >= 0)
+        val = bf16_to_f32(p.x[b * p.x_sb + t * p.x_st + ch]);
+      else if (p.conv_in != nullptr)
+        val = p.conv_in[(b * p.C + ch) * (KCONV - 1) + (KCONV - 1) + t];
+      p.conv_out[(b * p.C + ch) * (KCONV - 1) + s] = val;
+    }
+  }
   half_t* q_out = p.qn + ((b * p.Hk + hk) * p.nch + c) * (CH * DK);
   cfloat4 xd, xa[2], xq[2][2];
   if (wave == 0) blocks_gram<0>(smem, q_out, lane, xd, xa, xq);

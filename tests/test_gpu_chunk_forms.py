@@ -57,3 +57,55 @@ def test_forms_match_oracle(batch, key_heads, value_heads, seq) -> None:
 @pytest.mark.parametrize("seq", [2, 63, 192, 259])
 def test_split_form_unaligned_rows_and_fp32_output(batch, key_heads, value_heads, seq) -> None:
     _case(batch, key_heads, value_heads, seq, seq != 192, False, torch.float32)
+
+
+def _abi(x, a, b, a_log, dt_bias, w, key_heads, conv_in, conv_out, state_in, state_out, workspace) -> torch.Tensor:
+    """``qa_chunk_gated_delta_rule`` on the caller's own buffers, ``workspace`` of its own size."""
+    import ctypes
+
+    import hip_loader
+    import hip_ops
+
+    lib = hip_loader.load_library()
+    batch, seq, _ = x.shape
+    heads = a.shape[2]
+    out = torch.empty(batch, seq, heads, 128, dtype=torch.bfloat16, device=DEV)
+    ptr = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())  # noqa: E731
+    status = lib.qa_chunk_gated_delta_rule(
+        ptr(x), hip_loader.QA_BF16, x.stride(0), x.stride(1), ptr(a), ptr(b), hip_loader.QA_F32, a.stride(0), a.stride(1), ptr(a_log), ptr(dt_bias),
+        ptr(w), ptr(conv_in), ptr(conv_out), ptr(state_in), ptr(state_out), ptr(out), hip_loader.QA_BF16, out.stride(0), out.stride(1), batch, seq,
+        key_heads, heads, 128, 128, 4, ptr(workspace), workspace.numel(), hip_ops._stream(x.device))
+    hip_loader.check(lib, status, "chunk_gated_delta_rule")
+    return out
+
+
+def _device_inputs(batch: int, key_heads: int, value_heads: int, seq: int):
+    gen = torch.Generator().manual_seed(100 * batch + seq)
+    channels = 2 * key_heads * 128 + value_heads * 128
+    x = torch.randn(batch, seq, channels, generator=gen).to(torch.bfloat16).to(DEV)
+    a, b = (torch.randn(batch, seq, value_heads, generator=gen).to(DEV) for _ in range(2))
+    a_log, dt_bias = (torch.randn(value_heads, generator=gen) - 1.0).to(DEV), torch.zeros(value_heads, device=DEV)
+    w = (torch.randn(channels, 4, generator=gen) * 0.5).to(DEV)
+    tail = torch.randn(batch, channels, 3, generator=gen).to(DEV)
+    state = (0.05 * torch.randn(batch, value_heads, 128, 128, generator=gen)).to(DEV)
+    return x, a, b, a_log, dt_bias, w, tail, state
+
+
+def _workspace(batch: int, seq: int, key_heads: int, value_heads: int) -> torch.Tensor:
+    import hip_loader
+
+    size = hip_loader.load_library().qa_chunk_gated_delta_workspace(batch, seq, key_heads, value_heads)
+    return torch.empty(size, dtype=torch.uint8, device=DEV)
+
+
+@pytest.mark.parametrize("batch,key_heads,value_heads", [(1, 2, 4), (3, 1, 11), (5, 1, 13)])
+@pytest.mark.parametrize("seq", [1, 2, 3, 33])
+def test_states_updated_in_place(batch, key_heads, value_heads, seq) -> None:
+    x, a, b, a_log, dt_bias, w, tail, state = _device_inputs(batch, key_heads, value_heads, seq)
+    ws = _workspace(batch, seq, key_heads, value_heads)
+    new_tail, new_state = torch.empty_like(tail), torch.empty_like(state)
+    want = _abi(x, a, b, a_log, dt_bias, w, key_heads, tail, new_tail, state, new_state, ws)
+    out = _abi(x, a, b, a_log, dt_bias, w, key_heads, tail, tail, state, state, ws)
+    assert torch.equal(out, want)
+    assert torch.equal(tail, new_tail)
+    assert torch.equal(state, new_state)
