@@ -364,14 +364,18 @@ int qa_gated_delta_step_conv(const void* x, int32_t x_dtype, int64_t x_stride_b,
  * initial_state/final_state (B, Hv, dk, dv) fp32 (NULL in = zeros).
  * final_state may be initial_state; conv_state_out may be conv_state_in only
  * for T <= 33, beyond that waves that nothing orders read the one and write
- * the other.  Writes out (B, T, Hv, dv) float32/bfloat16.  Computes the conv1d + SiLU, L2 norm,
- * q scale and gating of src/reference_ops.py:240-283 and the recurrence of
- * :291-322 in 64-token chunks (WY/UT form) on fp16 MFMA with fp32
- * accumulation and an fp32 state.  dk = dv = 128, conv kernel 4.  The
- * workspace (256-byte aligned, qa_chunk_gated_delta_workspace bytes) holds the
- * normalised fp16 q/k and the gates between the launches (the v channels are
- * convolved inside the second launch).  The reference
- * has no chunked kernel: its prefill runs the token-serial recurrence
+ * the other.  Writes out (B, T, Hv, dv) float32/bfloat16.  Computes the
+ * conv1d + SiLU, L2 norm, q scale and gating of src/reference_ops.py:240-283
+ * and the recurrence of :291-322 in 64-token chunks (WY/UT form) on fp16 MFMA
+ * with fp32 accumulation and an fp32 state.  dk = dv = 128, conv kernel 4.
+ * The workspace (256-byte aligned, qa_chunk_gated_delta_workspace bytes) holds
+ * the normalised fp16 q/k between the two launches (the v channels are
+ * convolved inside the second one), and with them either the gates (16 bytes
+ * per token and value head) or, for few (row, value head) pairs, the operands
+ * of the state chain (17 KB per 64 tokens and value head).  A buffer too small
+ * for the latter is used for the former, so one sized for more rows, of the
+ * same T and heads, serves fewer rows too.  The reference has no chunked
+ * kernel: its prefill runs the token-serial recurrence
  * (src/tp_runtime.py:2744-2787).                                          */
 int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype, int64_t x_stride_b, int64_t x_stride_t,
                               const void* a, const void* b, int32_t ab_dtype, int64_t ab_stride_b, int64_t ab_stride_t,
@@ -383,8 +387,10 @@ int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype, int64_t x_
                               int32_t key_dim, int32_t value_dim, int32_t conv_kernel,
                               void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
-/* Workspace bytes qa_chunk_gated_delta_rule needs for these sizes (dk = dv = 128);
- * no counterpart in the reference, whose prefill keeps no intermediate buffers. */
+/* Workspace bytes of the form qa_chunk_gated_delta_rule takes for these sizes
+ * (dk = dv = 128).  Not monotonic in batch: where the form changes, one more
+ * row may ask for less (see above for reusing a buffer).  No counterpart in the
+ * reference, whose prefill keeps no intermediate buffers.                    */
 int64_t qa_chunk_gated_delta_workspace(int64_t batch, int64_t seq, int32_t key_heads, int32_t value_heads);
 
 /* LDS bytes one chunked-prefill workgroup reserves (for capacity planning). */

@@ -97,9 +97,11 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t{255}; }
 
 constexpr int64_t kRecBytes = 17 * 1024;  // record of the split form per (row, value head, chunk), see REC_BYTES
 
-inline Workspace workspace_layout(int64_t batch, int64_t seq, int64_t hk, int64_t hv) {
+inline bool split_form(int64_t batch, int64_t hv) { return batch * hv <= kSplitHeads; }
+
+inline Workspace workspace_layout(int64_t batch, int64_t seq, int64_t hk, int64_t hv, bool split) {
   Workspace w{};
-  w.split = batch * hv <= kSplitHeads;
+  w.split = split;
   w.nch = (seq + CH - 1) / CH;
   w.tp = w.nch * CH;
   const int64_t qk = batch * w.tp * hk * DK * 2;  // qn, kn: (B, Tp, Hk, 128), or tiles per (row, key head, chunk)
@@ -2161,7 +2163,7 @@ extern "C" int64_t qa_chunk_gated_delta_lds_bytes(void) { return qa::cgd::LDS_BY
 
 extern "C" int64_t qa_chunk_gated_delta_workspace(int64_t batch, int64_t seq, int32_t key_heads, int32_t value_heads) {
   if (batch <= 0 || seq <= 0 || key_heads <= 0 || value_heads <= 0) return 0;
-  return qa::cgd::workspace_layout(batch, seq, key_heads, value_heads).bytes;
+  return qa::cgd::workspace_layout(batch, seq, key_heads, value_heads, qa::cgd::split_form(batch, value_heads)).bytes;
 }
 
 extern "C" int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype, int64_t x_stride_b, int64_t x_stride_t,
@@ -2191,7 +2193,11 @@ extern "C" int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype,
   QA_REQUIRE(out_stride_t % 4 == 0 && out_stride_b % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0,
              "chunk_gated_delta_rule: output rows must be 16-byte aligned");
   QA_REQUIRE((reinterpret_cast<uintptr_t>(conv_weight) & 15u) == 0, "chunk_gated_delta_rule: conv_weight must be 16-byte aligned");
-  const Workspace ws = workspace_layout(batch, seq, key_heads, value_heads);
+  // The split form needs the larger workspace, so sizes do not grow with the batch across kSplitHeads (16 key and 32
+  // value heads, 8192 tokens: 277 MB for two rows, 214 MB for three).  A caller's buffer that was sized for more rows
+  // than this call has holds at least the layout of prep_kernel and chunk_kernel, which then run.
+  Workspace ws = workspace_layout(batch, seq, key_heads, value_heads, split_form(batch, value_heads));
+  if (workspace_bytes < ws.bytes) ws = workspace_layout(batch, seq, key_heads, value_heads, false);
   QA_REQUIRE(workspace != nullptr && workspace_bytes >= ws.bytes && (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
              "chunk_gated_delta_rule: workspace must be 256-byte aligned and hold %lld bytes", static_cast<long long>(ws.bytes));
   unsigned char* wsb = static_cast<unsigned char*>(workspace);

@@ -109,3 +109,23 @@ def test_states_updated_in_place(batch, key_heads, value_heads, seq) -> None:
     assert torch.equal(out, want)
     assert torch.equal(tail, new_tail)
     assert torch.equal(state, new_state)
+
+
+def test_workspace_sized_for_more_rows_serves_fewer() -> None:
+    # 64 (row, value head) pairs ask for more than 68: the larger batch's buffer holds only the unsplit form's layout
+    key_heads, value_heads, seq = 2, 4, 65
+    own, reused = _workspace(16, seq, key_heads, value_heads), _workspace(17, seq, key_heads, value_heads)
+    assert reused.numel() < own.numel()
+    x, a, b, a_log, dt_bias, w, tail, state = _device_inputs(16, key_heads, value_heads, seq)
+    args = (x, a, b, a_log, dt_bias, w, key_heads, tail)
+    results = []
+    for ws in (own, reused):
+        new_tail, new_state = torch.empty_like(tail), torch.empty_like(state)
+        results.append((_abi(*args, new_tail, state, new_state, ws), new_state, new_tail))
+    (want, want_state, want_tail), (out, new_state, new_tail) = results
+    torch.testing.assert_close(out.float(), want.float(), atol=2e-2, rtol=2e-2)
+    assert float((new_state - want_state).double().norm() / want_state.double().norm()) < 1e-3
+    assert torch.equal(new_tail, want_tail)
+    least = _workspace(17, seq, key_heads, value_heads).numel() * 16 // 17  # 16 rows of the unsplit layout, whole 256 bytes
+    with pytest.raises(RuntimeError, match="workspace"):
+        _abi(*args, None, state, None, reused[: least - 256])
