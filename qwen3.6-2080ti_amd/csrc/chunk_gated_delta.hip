@@ -97,7 +97,15 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t{255}; }
 
 constexpr int64_t kRecBytes = 17 * 1024;  // record of the split form per (row, value head, chunk), see REC_BYTES
 
-inline bool split_form(int64_t batch, int64_t hv) { return batch * hv <= kSplitHeads; }
+// blocks_kernel takes the value heads of a key head one after the other (1.1 us each), which long sequences hide
+// behind their chunks: the split form from (value heads per key head - kSplitGroup) chunks on.  Both sides measured (us,
+// unsplit : split): 8 a key head, 1 token 24 : 23; 16 a key head, 128 tokens 31 : 34, 512 tokens 46 : 45; 32 a key head,
+// 1000 tokens 66 : 73, 2048 tokens 108 : 91; 64 a key head, 2048 tokens 109 : 135, 4096 tokens 190 : 176.
+constexpr int64_t kSplitGroup = 8;
+
+inline bool split_form(int64_t batch, int64_t seq, int64_t hk, int64_t hv) {
+  return batch * hv <= kSplitHeads && hv / hk - kSplitGroup <= (seq + CH - 1) / CH;
+}
 
 inline Workspace workspace_layout(int64_t batch, int64_t seq, int64_t hk, int64_t hv, bool split) {
   Workspace w{};
@@ -2163,7 +2171,7 @@ extern "C" int64_t qa_chunk_gated_delta_lds_bytes(void) { return qa::cgd::LDS_BY
 
 extern "C" int64_t qa_chunk_gated_delta_workspace(int64_t batch, int64_t seq, int32_t key_heads, int32_t value_heads) {
   if (batch <= 0 || seq <= 0 || key_heads <= 0 || value_heads <= 0) return 0;
-  return qa::cgd::workspace_layout(batch, seq, key_heads, value_heads, qa::cgd::split_form(batch, value_heads)).bytes;
+  return qa::cgd::workspace_layout(batch, seq, key_heads, value_heads, qa::cgd::split_form(batch, seq, key_heads, value_heads)).bytes;
 }
 
 extern "C" int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype, int64_t x_stride_b, int64_t x_stride_t,
@@ -2196,7 +2204,7 @@ extern "C" int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype,
   // The split form needs the larger workspace, so sizes do not grow with the batch across kSplitHeads (16 key and 32
   // value heads, 8192 tokens: 277 MB for two rows, 214 MB for three).  A caller's buffer that was sized for more rows
   // than this call has holds at least the layout of prep_kernel and chunk_kernel, which then run.
-  Workspace ws = workspace_layout(batch, seq, key_heads, value_heads, split_form(batch, value_heads));
+  Workspace ws = workspace_layout(batch, seq, key_heads, value_heads, split_form(batch, seq, key_heads, value_heads));
   if (workspace_bytes < ws.bytes) ws = workspace_layout(batch, seq, key_heads, value_heads, false);
   QA_REQUIRE(workspace != nullptr && workspace_bytes >= ws.bytes && (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
              "chunk_gated_delta_rule: workspace must be 256-byte aligned and hold %lld bytes", static_cast<long long>(ws.bytes));

@@ -59,6 +59,12 @@ def test_split_form_unaligned_rows_and_fp32_output(batch, key_heads, value_heads
     _case(batch, key_heads, value_heads, seq, seq != 192, False, torch.float32)
 
 
+# either side of the line of the split form where a key head has many value heads: chunks = heads per key head - 8
+@pytest.mark.parametrize("batch,key_heads,value_heads,seq", [(1, 1, 10, 64), (1, 1, 10, 65), (2, 1, 12, 192), (2, 1, 12, 193)])
+def test_many_value_heads_per_key_head_match_oracle(batch, key_heads, value_heads, seq) -> None:
+    _case(batch, key_heads, value_heads, seq, True, True, torch.bfloat16)
+
+
 def _abi(x, a, b, a_log, dt_bias, w, key_heads, conv_in, conv_out, state_in, state_out, workspace) -> torch.Tensor:
     """``qa_chunk_gated_delta_rule`` on the caller's own buffers, ``workspace`` of its own size."""
     import ctypes
