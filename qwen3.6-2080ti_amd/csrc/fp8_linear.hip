@@ -939,32 +939,11 @@ struct Plan {
   int64_t workspace;      // partials, then (rows >= 16) the fp16 copy of an fp32 x
 };
 
-// Rows per workgroup and the K split, from the shape alone (so the workspace query and
+// The plan without the block path.  Rows per workgroup and the K split, from the shape alone (so the workspace query and
 // the launch agree): K is split only when there are fewer than 256 tiles, to about 256
 // workgroups with at least four K blocks each.
-inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
+inline Plan make_row_plan(int64_t M, int64_t N, int64_t K) {
   Plan pl{};
-  // Block path: the largest tile that gives at least 192 of the 256 CUs a workgroup (160 for the smallest, whose
-  // workgroups are short), up to 128 rows the x-resident and wide kernels.  Both sides measured (us, fp32 x, packed):
-  // 128 x 256 against 128 x 128 at 192 tiles (768 x 8192 x 2048) 38.6 : 44.8, at 128 tiles (1024 x 4096 x 2048) 35.5 : 29.4;
-  // 128 x 128 against 64 x 128 at 192 tiles (768 x 4096 x 2048) 26.5 : 27.0, at 128 tiles (1024 x 2048 x 4096) 39.9 : 34.7;
-  // 64 x 128 against the paths below at 160 tiles (300 x 4096 x 2048) 19.2 : 27.2, at 128 tiles (512 x 2048 x 4096)
-  // 31.5 : 29.0 and (256 x 4096 x 2048) 19.0 : 14.2.
-  if (M > 128) {
-    const int64_t tm = (M + 127) / 128, tn = N / 128;
-    pl.block = tm * ((tn + 1) / 2) >= 192 ? 1 : tm * tn >= 192 ? 2 : (M + 63) / 64 * tn >= 160 ? 3 : 0;
-  }
-  if (pl.block) {
-    // bf16 rows too far apart for 32-bit offsets: the wide kernel
-    pl.wide = 1;
-    pl.xt = 4;
-    pl.mtiles = (M + 63) / 64;
-    pl.ntiles = N / WN;
-    pl.ksplit = 1;
-    pl.blocks_per_split = static_cast<int>(K / KB);
-    pl.workspace = M * K * 2;  // the fp16 copy of an fp32 x
-    return pl;
-  }
   if (M > 16 && M <= 256 && K <= XR_KMAX) {
     // x is 16-bit here in both input dtypes (fp32 x of 16 rows or more is cast to fp16 first)
     pl.xres = 1;
@@ -997,6 +976,33 @@ inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
   pl.ksplit = static_cast<int>((kblocks + pl.blocks_per_split - 1) / pl.blocks_per_split);
   pl.partial_bytes = pl.ksplit > 1 ? (static_cast<int64_t>(pl.ksplit) * M * N * 4 + 255) / 256 * 256 : 0;
   pl.workspace = pl.partial_bytes + (M >= 16 ? M * K * 2 : 0);
+  return pl;
+}
+
+inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
+  Plan pl = make_row_plan(M, N, K);
+  // Block path: the largest tile that gives at least 192 of the 256 CUs a workgroup (160 for the smallest, whose
+  // workgroups are short), up to 128 rows the x-resident and wide kernels.  Both sides measured (us, fp32 x, packed):
+  // 128 x 256 against 128 x 128 at 192 tiles (768 x 8192 x 2048) 38.6 : 44.8, at 128 tiles (1024 x 4096 x 2048) 35.5 : 29.4;
+  // 128 x 128 against 64 x 128 at 192 tiles (768 x 4096 x 2048) 26.5 : 27.0, at 128 tiles (1024 x 2048 x 4096) 39.9 : 34.7;
+  // 64 x 128 against the paths below at 160 tiles (300 x 4096 x 2048) 19.2 : 27.2, at 128 tiles (512 x 2048 x 4096)
+  // 31.5 : 29.0 and (256 x 4096 x 2048) 19.0 : 14.2.
+  if (M > 128) {
+    const int64_t tm = (M + 127) / 128, tn = N / 128;
+    pl.block = tm * ((tn + 1) / 2) >= 192 ? 1 : tm * tn >= 192 ? 2 : (M + 63) / 64 * tn >= 160 ? 3 : 0;
+  }
+  if (pl.block) {
+    // bf16 rows too far apart for 32-bit offsets: the wide kernel
+    pl.xres = 0;
+    pl.wide = 1;
+    pl.xt = 4;
+    pl.mtiles = (M + 63) / 64;
+    pl.ntiles = N / WN;
+    pl.ksplit = 1;
+    pl.blocks_per_split = static_cast<int>(K / KB);
+    pl.partial_bytes = 0;
+    pl.workspace = M * K * 2;  // the fp16 copy of an fp32 x
+  }
   return pl;
 }
 
@@ -1061,7 +1067,10 @@ void launch(const Plan& pl, const Params& p, int mode, hipStream_t stream) {
 
 extern "C" int64_t qa_fp8_linear_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
   if (rows <= 0 || out_features <= 0 || in_features <= 0 || out_features % 128 != 0 || in_features % 128 != 0) return 0;
-  return qa::f8l::make_plan(rows, out_features, in_features).workspace;
+  // what the paths without the block kernel need, never less than it does: a caller's buffer for one row count then holds
+  // fewer rows of the same weight too where the larger count takes the block kernel and the smaller one splits K
+  // (2048 x 2048: 13.1 MB for 640 rows, of which the block kernel uses 2.6, 10.5 MB for 512)
+  return qa::f8l::make_row_plan(rows, out_features, in_features).workspace;
 }
 
 extern "C" int qa_fp8_pack_weight(const void* weight, void* packed, int64_t out_features, int64_t in_features, hipStream_t stream) {

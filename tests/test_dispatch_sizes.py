@@ -28,3 +28,11 @@ def _chunk_workspace(batch: int, seq: int, key_heads: int, value_heads: int, spl
 def test_chunked_delta_rule_form(batch, seq, key_heads, value_heads, split) -> None:
     size = _library().qa_chunk_gated_delta_workspace(batch, seq, key_heads, value_heads)
     assert size == _chunk_workspace(batch, seq, key_heads, value_heads, split)
+
+
+@pytest.mark.parametrize("out_features,in_features", [(2048, 2048), (2048, 4096)])
+def test_fp8_linear_workspace_of_more_rows_holds_fewer(out_features, in_features) -> None:
+    # 512 to 960 rows: without the block kernel all of them split K in two, with it the larger counts do not split
+    sizes = [_library().qa_fp8_linear_workspace(rows, out_features, in_features) for rows in range(512, 961, 32)]
+    assert sizes == sorted(sizes)
+    assert sizes[0] >= 2 * 512 * out_features * 4 + 512 * in_features * 2  # fp32 partials, then x as fp16
