@@ -992,14 +992,8 @@ inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
     pl.block = tm * ((tn + 1) / 2) >= 192 ? 1 : tm * tn >= 192 ? 2 : (M + 63) / 64 * tn >= 160 ? 3 : 0;
   }
   if (pl.block) {
-    // bf16 rows too far apart for 32-bit offsets: the wide kernel
-    pl.xres = 0;
-    pl.wide = 1;
-    pl.xt = 4;
-    pl.mtiles = (M + 63) / 64;
-    pl.ntiles = N / WN;
+    pl.xres = pl.wide = 0;
     pl.ksplit = 1;
-    pl.blocks_per_split = static_cast<int>(K / KB);
     pl.partial_bytes = 0;
     pl.workspace = M * K * 2;  // the fp16 copy of an fp32 x
   }
@@ -1107,7 +1101,9 @@ extern "C" int qa_fp8_linear(const void* x, int32_t x_dtype, int64_t x_stride, i
   const int ysize = y_dtype == QA_F32 ? 4 : 2;
   QA_REQUIRE((reinterpret_cast<uintptr_t>(y) & 15u) == 0 && (y_stride * ysize) % 16 == 0, "output rows must be 16-byte aligned");
   QA_REQUIRE(rows <= 0x7fffffffLL * 16 && out_features / 128 <= 0x7fffffff, "shape too large");
-  const Plan pl = make_plan(rows, out_features, in_features);
+  // bf16 rows too far apart for the block kernel's 32-bit offsets (fp32 rows reach it as a contiguous copy)
+  const bool far = x_dtype == QA_BF16 && x_stride > kBlockMaxStride;
+  const Plan pl = far ? make_row_plan(rows, out_features, in_features) : make_plan(rows, out_features, in_features);
   QA_REQUIRE(pl.mtiles <= 65535, "fp8_linear: too many rows (%lld)", static_cast<long long>(rows));
   QA_REQUIRE(pl.workspace == 0 || (workspace != nullptr && workspace_bytes >= pl.workspace && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0),
              "fp8_linear: workspace must hold %lld bytes", static_cast<long long>(pl.workspace));
@@ -1154,7 +1150,7 @@ extern "C" int qa_fp8_linear(const void* x, int32_t x_dtype, int64_t x_stride, i
     if (rc) return rc;
     return check_launch("fp8_linear");
   }
-  if (pl.block && p.x_stride <= kBlockMaxStride) {
+  if (pl.block) {
     int rc = 0;
     {
       KernelTimer timer_("fp8_linear", stream);

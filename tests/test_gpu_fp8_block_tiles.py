@@ -61,13 +61,27 @@ def test_nan_code_and_infinite_row_stay_in_their_column_and_row() -> None:
     assert torch.isfinite(out[:299, :8191]).all().item()
 
 
-def test_rows_further_apart_than_the_block_kernel_takes() -> None:
+# The largest row stride that the block kernel takes and the next one past it, through the C ABI (the Python entry makes
+# x contiguous first): past it the x-resident, wide and tiled kernels (in_features 128 and 2176; up to 256 rows and more)
+# and a K split (in_features 2176, 5 x 32 tiles).
+@pytest.mark.parametrize("rows,n,k", [(129, 8192, 128), (129, 8192, 2176), (257, 4096, 2176), (385, 4096, 128)])
+@pytest.mark.parametrize("past", [0, 8])
+def test_rows_further_apart_than_the_block_kernel_takes(rows, n, k, past) -> None:
+    import ctypes
+
+    import hip_loader
     import hip_ops as ops
 
-    x, w, s = _inputs(129, 8192, 128, torch.bfloat16)
-    stride = (1 << 23) + 8
-    far = torch.as_strided(torch.empty(128 * stride + 128, dtype=torch.bfloat16, device=DEV), (129, 128), (stride, 1))
-    far.copy_(x.to(DEV))
-    out = ops.fp8_e4m3_bf16_linear(far, w.to(DEV), s.to(DEV))
+    stride = (1 << 23) + past
+    x, w, s = _inputs(rows, n, k, torch.bfloat16)
+    xd, wd, sd = torch.empty((rows - 1) * stride + k, dtype=torch.bfloat16, device=DEV).as_strided((rows, k), (stride, 1)), w.to(DEV), s.to(DEV)
+    xd.copy_(x.to(DEV))
+    lib = hip_loader.load_library()
+    workspace = torch.empty(lib.qa_fp8_linear_workspace(rows, n, k), dtype=torch.uint8, device=DEV)
+    out = torch.empty(rows, n, device=DEV)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    status = lib.qa_fp8_linear(ptr(xd), hip_loader.QA_BF16, stride, rows, ptr(wd), 0, ptr(sd), n, k, ptr(out), hip_loader.QA_F32, n, ptr(workspace),
+                               workspace.numel(), ops._stream(out.device))
+    hip_loader.check(lib, status, "fp8_linear")
     ref = _fp64(x, w, s)
     torch.testing.assert_close(out.cpu().double(), ref, atol=1e-5 * ref.abs().max().item(), rtol=1e-3)
