@@ -979,17 +979,30 @@ inline Plan make_row_plan(int64_t M, int64_t N, int64_t K) {
   return pl;
 }
 
+// Time of n equal workgroups, `per_round` of them at once on the 256 CUs: `full` for each full round and for what is left
+// over from `lone` (a few of them) towards `full`.  In us at in_features 2048; only the ratios matter.
+inline int64_t rounds_time(int64_t n, int64_t per_round, int64_t full, int64_t lone) {
+  const int64_t left = n % per_round;
+  return n / per_round * full + (left ? lone + (full - lone) * left / per_round : 0);
+}
+
+// Block path: from 160 tiles of 64 x 128 on, up to 256 rows and beyond (fewer: 512 x 2048 x 4096, 128 tiles, 31.5 us
+// against 29.0 below; 256 x 4096 x 2048 19.0 against 14.2), with the tile that takes the least time by whole rounds: the
+// 128-row tiles have a CU to themselves, of the 64-row ones two share it.  A tile count just past a round costs almost a
+// round, so the largest tile that fills the chip is not the fastest.  Measured (us, fp32 x, packed weight, tiles of
+// 128 x 256 : 128 x 128 : 64 x 128): 513 x 8192 x 2048 34.1 : 41.8 : 37.5; 1025 x 4096 x 2048 34.8 : 43.9 : 38.7;
+// 300 x 12288 x 4096 51.3 : 72.2 : 44.9 (tiled path 50.7); 385 x 9216 x 4096 51.8 : 72.8 : 46.2 (51.5);
+// 1281 x 6144 x 2048 66.7 : 64.5 : 50.6 (57.8); 384 x 8192 x 2048 31.5 : 25.0 : 25.1; 1024 x 8192 x 2048
+// 42.9 : 49.4 : 50.8; 300 x 4096 x 2048 29.4 : 22.1 : 18.5.  Of 198 sizes measured the
+// rule's tile is within 11% of the fastest of the three.
 inline Plan make_plan(int64_t M, int64_t N, int64_t K) {
   Plan pl = make_row_plan(M, N, K);
-  // Block path: the largest tile that gives at least 192 of the 256 CUs a workgroup (160 for the smallest, whose
-  // workgroups are short), up to 128 rows the x-resident and wide kernels.  Both sides measured (us, fp32 x, packed):
-  // 128 x 256 against 128 x 128 at 192 tiles (768 x 8192 x 2048) 38.6 : 44.8, at 128 tiles (1024 x 4096 x 2048) 35.5 : 29.4;
-  // 128 x 128 against 64 x 128 at 192 tiles (768 x 4096 x 2048) 26.5 : 27.0, at 128 tiles (1024 x 2048 x 4096) 39.9 : 34.7;
-  // 64 x 128 against the paths below at 160 tiles (300 x 4096 x 2048) 19.2 : 27.2, at 128 tiles (512 x 2048 x 4096)
-  // 31.5 : 29.0 and (256 x 4096 x 2048) 19.0 : 14.2.
-  if (M > 128) {
-    const int64_t tm = (M + 127) / 128, tn = N / 128;
-    pl.block = tm * ((tn + 1) / 2) >= 192 ? 1 : tm * tn >= 192 ? 2 : (M + 63) / 64 * tn >= 160 ? 3 : 0;
+  const int64_t tm = (M + 127) / 128, tn = N / 128, small = (M + 63) / 64 * tn;
+  if (M > 128 && small >= 160) {
+    const int64_t t1 = rounds_time(tm * ((tn + 1) / 2), 256, 34, 18);
+    const int64_t t2 = rounds_time(tm * tn, 256, 20, 15);
+    const int64_t t3 = rounds_time(small, 512, 21, 11);
+    pl.block = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
   }
   if (pl.block) {
     pl.xres = pl.wide = 0;

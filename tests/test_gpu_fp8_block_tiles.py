@@ -29,10 +29,12 @@ def _fp64(x: torch.Tensor, w: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
     return x.double() @ full.t()
 
 
-# tiles of 64 x 128, 128 x 128 and 128 x 256, the first sizes past each line of the rule among them; out_features
-# that leave half a tile; one K block (two stages, fewer than the ring) and an odd number of them
+# tiles of 64 x 128, 128 x 128 and 128 x 256, sizes either side of where the rule changes tile among them; counts of
+# tiles just past a whole round; out_features that leave half a tile; one K block (two stages, fewer than the ring) and
+# an odd number of them
 @pytest.mark.parametrize("rows,n,k", [(129, 8192, 128), (192, 8192, 384), (193, 6912, 128), (257, 8192, 256), (300, 4096, 640), (385, 8064, 128),
-                                      (641, 8192, 128), (769, 7296, 384), (767, 4096, 128), (4097, 1664, 128), (2560, 512, 256)])
+                                      (641, 8192, 128), (769, 7296, 384), (767, 4096, 128), (4097, 1664, 128), (2560, 512, 256), (300, 12288, 128), (513, 8192, 128),
+                                      (1281, 6144, 128)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_block_tiles_match_fp64(rows, n, k, dtype) -> None:
     import hip_ops as ops
