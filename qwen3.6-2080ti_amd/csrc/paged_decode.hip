@@ -616,9 +616,15 @@ __global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_balanced(De
 
 // The same merge with kSplitCombineWaves waves per (row, head), for row groups of many partials: bound by
 // the latency of its loads, so each wave merges a contiguous share, kSplitCombineRows rows in flight at a
-// time (64 registers: 16 waves a workgroup leave 128), and the waves' (m, l, o) meet in LDS.
+// time (64 registers: 16 waves a workgroup leave 128), and the waves' (m, l, o) meet in LDS.  The host knows
+// only the mean number of partials (see split_combine): a row group of up to kColumnCombineMax has its
+// columns shared by D / 64 waves instead, kColumnCombineRows rows in flight, with no barrier (us, 16 waves
+// and LDS : columns, decode_combine_balanced: 32 rows of 512 tokens on 1 x 128, 32 partials each,
+// 21.0 : 16.9, 16.4; 32 rows of 1024 to 8192 30.9 : 28.1, 28.7).
 constexpr int kSplitCombineWaves = 16;
 constexpr int kSplitCombineRows = 16;
+constexpr int kColumnCombineMax = 64;
+constexpr int kColumnCombineRows = 32;
 
 template <typename QT, int D>
 __global__ __launch_bounds__(64 * kSplitCombineWaves) void decode_combine_split(DecodeParams p) {
@@ -649,6 +655,31 @@ __global__ __launch_bounds__(64 * kSplitCombineWaves) void decode_combine_split(
   const int64_t sml = 2 * static_cast<int64_t>(p.G);
   const int64_t so = static_cast<int64_t>(p.G) * D;
 
+  if (n <= kColumnCombineMax) {
+    // few partials: wave w takes all of them for columns 64 w .. 64 w + 63, so no barrier; the other waves leave
+    if (wave >= CPL) return;
+    const float* col = p.part_o + (slot0 * p.G + hh) * D + 64 * wave + lane;
+    const float2 e = lane < n ? *reinterpret_cast<const float2*>(ml + lane * sml) : make_float2(-INFINITY, 0.f);
+    float rows[kColumnCombineRows];
+#pragma unroll
+    for (int s = 0; s < kColumnCombineRows; ++s) rows[s] = s < n ? col[s * so] : 0.f;
+    const float m = wave_max(e.x);
+    const float f = lane < n ? exp2f(e.x - (m == -INFINITY ? 0.f : m)) : 0.f;
+    const float l = wave_sum(f * e.y);
+    float o = 0.f;
+#pragma unroll
+    for (int s = 0; s < kColumnCombineRows; ++s)
+      if (s < n) o += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), s)) * rows[s];
+    if (n > kColumnCombineRows) {
+#pragma unroll
+      for (int s = 0; s < kColumnCombineRows; ++s) rows[s] = kColumnCombineRows + s < n ? col[(kColumnCombineRows + s) * so] : 0.f;
+#pragma unroll
+      for (int s = 0; s < kColumnCombineRows; ++s)
+        if (kColumnCombineRows + s < n) o += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), kColumnCombineRows + s)) * rows[s];
+    }
+    Elem<QT>::store(out + 64 * wave + lane, l > 0.f ? o / l : 0.f);
+    return;
+  }
   const int end = n * (wave + 1) / kSplitCombineWaves;
   float m_run = -INFINITY, den = 0.f;
   vec_t acc = vec_t(0.f);
@@ -786,8 +817,9 @@ static int64_t decode_waves(int64_t row_groups, int64_t max_tokens) {
 
 // Which merge: from a mean of 32 partials a row group, as many as a wave of decode_combine_balanced has
 // in flight, the workgroup of decode_combine_split (4 rows of 100 to 8192 tokens 24.4 against 45.3 us, 8
-// of 700 to 4096 with D 128 17.7 against 21.7); below, its barrier and its 16 waves a head cost more than
-// they save (4 rows of 512, 16 partials: 17.2 against 15.7; 32 rows of 100 to 2048: 30.9 against 26.3).
+// of 700 to 4096 with D 128 17.7 against 21.7; 16 rows, one of 8192 tokens and the others of 100, 25.5
+// against 58); below, its 16 waves a head cost more than they save (4 rows of 512, 16 partials, on 2 x 256:
+// 17.2 against 15.7).
 static bool split_combine(const DecodeParams& p) { return p.n_waves >= 32 * static_cast<int64_t>(p.B) * p.Hkv; }
 
 // Bytes of workspace either path may need.  The generic path stores

@@ -1,7 +1,10 @@
 """Batched decode with few row groups against the CPU oracle: short chains, both merges, tables wider than the contexts.
 
-The launch has ``min(1024, tiles / 2)`` waves for up to 64 row groups, and the merge takes a workgroup per head
-from 32 partials a row group.  Tolerance for bf16 outputs as in the other decode tests: ``atol = rtol = 2e-2``.
+For up to 64 row groups the launch has a wave for every two tiles of the full tables, up to 1024 waves and at most 512 a
+row group (16 where there are more than 16 row groups); for more a wave for every eight.  With fewer tiles than waves
+each tile has a wave.  The merge takes a workgroup per head from a mean of 32 launched waves a row group, which shares
+the columns of up to 64 partials and the partials themselves above.  Tolerance for bf16 outputs as in the other decode
+tests: ``atol = rtol = 2e-2``.
 """
 
 from __future__ import annotations
@@ -44,6 +47,10 @@ def _case(lens, heads, kv_heads, dim, width, index, seed):
         ([512] * 4, 16, 2, 256, 0, torch.int32),  # 16 partials a row group: wave merge
         ([1023], 16, 2, 256, 0, torch.int32),  # 32 partials: workgroup merge
         ([8191], 16, 1, 128, 0, torch.int32),  # 256 partials, one row group
+        ([512], 16, 1, 256, 512, torch.int32),  # 32 partials, all in flight at once
+        ([528], 16, 2, 256, 512, torch.int32),  # 33
+        ([1024], 8, 1, 128, 512, torch.int32),  # 64, the last whose columns are shared
+        ([1040], 8, 1, 256, 512, torch.int32),  # 65
         ([4000, 1, 15, 16, 2047], 8, 2, 128, 0, torch.int64),  # skewed rows
         ([300 + 7 * r for r in range(17)], 8, 2, 128, 0, torch.int32),  # 34 row groups
         ([200 + 3 * r for r in range(33)], 4, 2, 128, 0, torch.int32),  # 66 row groups: past the rule
