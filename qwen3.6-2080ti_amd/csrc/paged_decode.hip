@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256, QA_DECODE_WAVES_PER_SIMD) void decode_partial_
   // first, so on as many CUs as there are (us, on the first T / 4 workgroups : on all, 16 heads on 2 x 256: 16
   // rows of 100 tokens in tables of 2048 blocks 14.2 : 12.6, 8 rows of 512 in tables of 128 blocks 15.8 : 14.5).
   const int64_t W = min64(p.n_waves, T);
-  const int64_t wid = T < p.n_waves ? static_cast<int64_t>(wave) * gridDim.x + blockIdx.x : static_cast<int64_t>(blockIdx.x) * kMfmaWaves + wave;
+  const int64_t wid = T < p.n_waves ? static_cast<int64_t>(wave) * (p.n_waves / kMfmaWaves) + blockIdx.x : static_cast<int64_t>(blockIdx.x) * kMfmaWaves + wave;
   if (wid >= W) return;
   const int64_t lo = T * wid / W;
   const int64_t hi = T * (wid + 1) / W;
