@@ -171,8 +171,8 @@ int qa_paged_kv_gather(const qa_paged_kv* kv, int32_t head_dim, int64_t batch,
  * rows enters as a bf16 hi + lo pair (the reference's fp32 matvec regime),
  * of 16 rows or more rounded to fp16 (its fp16 GEMM regime, .cu:1411-1460); bf16
  * x as itself.  weight_packed = 1: weight is in qa_fp8_pack_weight's
- * order (same bytes, streamed contiguously).  workspace: qa_fp8_linear_workspace(rows, out, in) bytes
- * (0 when no K split is used; then it may be NULL).  Replaces
+ * order (same bytes, streamed contiguously).  workspace: qa_fp8_linear_workspace(rows, out, in) bytes,
+ * 16-byte aligned (0 below 16 rows without a K split; then it may be NULL).  Replaces
  * fp8_e4m3_bf16_linear (src/fp8_cuda.py:16-17 -> src/csrc/fp8_linear.h,
  * src/csrc/fp8_linear_cuda.cu:1368-1466) and the dequantised F.linear of
  * src/reference_ops.py:436-506.                                            */
@@ -393,7 +393,8 @@ int qa_chunk_gated_delta_rule(const void* mixed_qkv, int32_t x_dtype, int64_t x_
  * reference, whose prefill keeps no intermediate buffers.                    */
 int64_t qa_chunk_gated_delta_workspace(int64_t batch, int64_t seq, int32_t key_heads, int32_t value_heads);
 
-/* LDS bytes one chunked-prefill workgroup reserves (for capacity planning). */
+/* LDS bytes one chunked-prefill workgroup reserves, the most of any form (for
+ * capacity planning).                                                       */
 int64_t qa_chunk_gated_delta_lds_bytes(void);
 
 /* ---- linear-attention output stage: gated RMSNorm + SiLU(z) ---------------- */

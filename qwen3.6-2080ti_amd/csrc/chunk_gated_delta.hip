@@ -2,7 +2,7 @@
 // chunk 64), from the raw in_proj outputs of a linear-attention layer.
 //
 // Two launches on the caller's stream, in one of two forms chosen by the number of (row, value head)
-// pairs (kSplitHeads): prep_kernel and chunk_kernel, described here (steps 1 and 2 share one grid), or
+// pairs (split_form) and by what the workspace holds: prep_kernel and chunk_kernel, described here (steps 1 and 2 share one grid), or
 // for few pairs blocks_kernel and chain_kernel, the same arithmetic split at the state dependence
 // (described at blocks_kernel below).
 //  1. prep_kernel -- causal conv1d + SiLU of every q/k channel and the L2
@@ -80,7 +80,9 @@ constexpr int RUN = 11 * PU;  // tokens one prep wave walks (swept: 33 beats 21,
 // and chunk_kernel.  chunk_kernel runs two workgroups per (row, value head), each with the whole chain of its chunks
 // (about 2.5 us a chunk), so below 128 (row, value head) pairs it leaves CUs idle; the split form spreads the
 // state-independent work over all CUs and shortens the chain, at the price of writing that work's operands to HBM
-// and reading them back (36 KB per chunk and key head with two value heads, where chunk_kernel's prep writes 32).
+// and reading them back (66 KB per chunk and key head with two value heads: q and k tiles and two records; prep and
+// gating write 34) and of twice the workspace.  chain_kernel<2> covers 64 pairs in one round of its workgroups, one to
+// a CU; 128 pairs are two rounds of the whole chain.
 // Measured in us, linear_attention_prefill of 16 key heads, chunk_kernel against split: 32 pairs (one row of 32 value
 // heads) at 4096 tokens 216 : 124, at 1000 tokens 78 : 47; 64 pairs at 4096 tokens 240 : 198 (two rows of 32) and
 // 262 : 242 (four rows of 16); 96 pairs 153 : 147 at 2048 tokens and 331 : 352 at 5000; 128 pairs at 2048 173 : 186.
@@ -1214,10 +1216,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
 // ---------------------------------------------------------------------------
 // Split form: blocks_kernel does everything that does not depend on the state, for all chunks of all
 // heads at once on all CUs, and chain_kernel runs only the state chain, 16 or 32 dv columns to a
-// workgroup.  kSplitHeads says when, with both forms' times.
+// workgroup.  kSplitHeads and kSplitGroup say when, with both forms' times.
 //
 // Measured on an MI355X at one row of 6001 tokens, 16 key and 32 value heads (prep_kernel 34 us +
-// chunk_kernel 240 us there): blocks_kernel 41 us, 1.25 us a chunk for chain_kernel<1>, 118-129 us.
+// chunk_kernel 240 us there): blocks_kernel 38-40 us, 1.25 us a chunk for chain_kernel<1>, 116-121 us.
 // blocks_kernel is bound by HBM and VALU together: at 4 x 8192 tokens it moves 819 MB in 177 us,
 // 4.6 TB/s (224 us with 55 KB of LDS and two workgroups per CU instead of four).  chain_kernel is bound
 // by one wave's instruction issue and latencies per chunk (about 2700 cycles): timing copies without the
@@ -2167,6 +2169,7 @@ static int launch_chain(const ChainParams& p, int64_t slices, hipStream_t stream
 }  // namespace cgd
 }  // namespace qa
 
+static_assert(qa::cgd::Chain<2>::BYTES <= qa::cgd::LDS_BYTES, "the most of any form");
 extern "C" int64_t qa_chunk_gated_delta_lds_bytes(void) { return qa::cgd::LDS_BYTES; }
 
 extern "C" int64_t qa_chunk_gated_delta_workspace(int64_t batch, int64_t seq, int32_t key_heads, int32_t value_heads) {

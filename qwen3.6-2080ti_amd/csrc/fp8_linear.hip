@@ -23,10 +23,10 @@
 // K blocks.  Per K block the x tile goes to LDS (double-buffered, one barrier per
 // block); each wave streams its 32 weight rows straight from global memory into
 // registers two blocks ahead.  When the grid is small, K is split over workgroups
-// that write fp32 partials, summed in a fixed order by a second kernel.  Wide path
-// (17 to 256 rows of 16-bit x): see fp8_linear_wide_kernel below, one pass over K
-// per output tile with no K split.  Block path (many output tiles): see
-// fp8_linear_block_kernel.
+// that write fp32 partials, summed in a fixed order by a second kernel.  X-resident and wide
+// paths (17 to 256 rows of 16-bit x, above 128 where the block path has too few tiles): see
+// fp8_linear_xres_kernel and fp8_linear_wide_kernel below, one pass over K per output tile
+// with no K split.  Block path (more than 128 rows, many output tiles): see fp8_linear_block_kernel.
 #include "qa_common.h"
 
 #include <type_traits>
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void fp8_pack_kernel(const uint8_t* __restrict
   *reinterpret_cast<u32x4_v*>(dst + 16 * piece) = *reinterpret_cast<const u32x4_v*>(src + row * K + col);
 }
 
-// ---- Wide path (16-bit x of more than 16 rows): one pass over K per output tile.
+// ---- Wide path (17 to 256 rows of 16-bit x, in_features above XR_KMAX): one pass over K per output tile.
 //
 // Work item: 64 weight rows x 16 XT rows of x x all of K, 8 waves: wave w multiplies weight tile
 // w % 4 (16 rows) with x tiles [XT/2 (w / 4), XT/2 (w / 4 + 1)), so the two waves of a SIMD (w and
@@ -663,18 +663,18 @@ __global__ __launch_bounds__(WNT) void fp8_linear_xres_kernel(Params p) {
 // (global_load_lds_dwordx4) through a ring of four, three in flight.  The two waves of a SIMD (w and w + 4) work half a
 // stage apart: while one multiplies its 16 MFMAs the other reads the next operands from LDS and decodes the weights, and
 // a barrier at each change keeps them so; in step with each other both would wait for LDS at once and then both for the
-// matrix cores (4096 x 8192 x 2048: 169 us).  The copies and the scale FMAs of finished tiles are issued between the
+// matrix cores (4096 x 8192 x 2048: 168 us instead of 148).  The copies and the scale FMAs of finished tiles are issued between the
 // MFMAs.  A tile is summed over the 128 columns of a block before the block scale multiplies it into the accumulators.
-// The copies take a uniform base and a 32-bit lane offset: with a 64-bit address per lane each one waited for the MFMAs
-// of the SIMD's other wave (129 against 65 cycles; the whole product 184 us instead of 163).
+// The copies take a uniform base and a 32-bit lane offset: with a 64-bit address per lane the same product takes 151 us.
 // 16-byte pieces are XOR-swizzled by row (x: piece ^ row / 2 mod 8 of 128-byte rows, row-major weights: piece ^ row / 4
 // mod 4 of 64-byte rows; packed weights keep their order), so the lanes of one LDS access fall on distinct banks.  x is
 // the A operand: a lane's accumulators are one output column and a store instruction writes two 128-byte row pieces.
 // Workgroups go to the XCDs in contiguous ranges of tiles ordered by groups of kGroupN weight tiles, x tiles fastest
 // inside a group, so an XCD's L2 holds the group's weights while x streams.
 // What bounds it: an MFMA phase takes about 750 cycles for 520 cycles of MFMA (rows 4096, tile 128 x 256).  Measured
-// with fp32 x, its cast included (us, before: the tiled or x-resident kernels): 4096 x 8192 x 2048 208 -> 154 (895
-// TFLOP/s), 4096 x 2048 x 4096 110 -> 82, 1024 x 4096 x 2048 34.7 -> 29.4, 256 x 8192 x 2048 25.8 -> 20.6.
+// with fp32 x, its cast included, back to back in a graph (us, before: the tiled or x-resident kernels): 4096 x 8192 x
+// 2048 216 -> 148 (the kernel alone 138 to 148 by trace, 930 to 995 TFLOP/s), 4096 x 2048 x 4096 105 -> 78,
+// 1024 x 4096 x 2048 35.5 -> 29.4, 256 x 8192 x 2048 23.9 -> 19.5.
 typedef float f32x16_v __attribute__((ext_vector_type(16)));
 constexpr int kGroupN = 4;
 
