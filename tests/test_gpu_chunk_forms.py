@@ -1,7 +1,8 @@
 """Both forms of the chunked delta rule and both widths of the split form's workgroups, at their edges.
 
 The number of (row, value head) pairs picks the form: up to 32 pairs one 16-column slice per
-workgroup, up to 64 two, above that ``chunk_kernel``.  Each at sequence lengths around the conv
+workgroup, up to 64 two, above that ``chunk_kernel``, which also takes short sequences of more than
+eight value heads per key head.  Each at sequence lengths around the conv
 history (3 tokens) and the 64-token chunk, with odd and even chunk counts, with and without
 carried states, and with token rows that are only 4-byte aligned.  Tolerances as in
 ``test_gpu_chunk_gated_delta``: outputs 2e-2, fp32 state 1e-3 relative, conv state bit-exact.
@@ -104,7 +105,7 @@ def _workspace(batch: int, seq: int, key_heads: int, value_heads: int) -> torch.
     return torch.empty(size, dtype=torch.uint8, device=DEV)
 
 
-@pytest.mark.parametrize("batch,key_heads,value_heads", [(1, 2, 4), (3, 1, 11), (5, 1, 13)])
+@pytest.mark.parametrize("batch,key_heads,value_heads", [(1, 2, 4), (3, 4, 12), (5, 1, 13)])
 @pytest.mark.parametrize("seq", [1, 2, 3, 33])
 def test_states_updated_in_place(batch, key_heads, value_heads, seq) -> None:
     x, a, b, a_log, dt_bias, w, tail, state = _device_inputs(batch, key_heads, value_heads, seq)
